@@ -779,12 +779,13 @@ static int cycle_fields(gev_ctx *c, const gev_sim_params *p, const gev_cycle_sta
         if (!rc) rc = launch_zsolve_vector(c, c->BiFT, zout_b, fourpiG * dx * dx, 0., c->BiFT);
     } else {
         rc = launch_zsolve_tensor(c, c->SijFT, zout_chi, a * a * st->dtau_old, true, nullptr, chik0);
-        if (!rc) rc = fft_backward_yx(c, zout_chi, c->chi, 1);
+        // chi and, in a GR run, B in the same launches
+        if (!rc) rc = fft_backward_yx(c, zout_chi, c->chi, p->gr_flag > 0 ? 4 : 1, Batch{}, c->Bi);
     }
     if (rc) return rc;
     // scalarFT ends the cycle holding chi(k=0) in both forms
     if (c->fp32 && (rc = launch_convert(c, chik0, false, c->scalarFT, true, 2))) return rc;
-    if (p->gr_flag > 0) {
+    if (p->vector_flag == 1 && p->gr_flag > 0) {
         rc = fft_backward_yx(c, zout_b, c->Bi, 3);
         if (rc) return rc;
     }

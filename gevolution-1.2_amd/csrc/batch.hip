@@ -285,12 +285,11 @@ int field_stage(gev_batch *B) {
         if (!rc) rc = fft_backward_yx(c, c->fft_tmp, c->phi, 1, phi);
     }
     if (rc) return rc;
-    double2 *const zout_chi = c->SijFT, *const zout_b = kcomp(c, c->SijFT, 1);
     rc = launch_x_prep_tensor(c, 0., all);
     if (!rc) rc = fft_forward_y(c, c->SijFT, 6, all);
-    if (!rc) rc = launch_zsolve_tensor(c, c->SijFT, zout_chi, 0., true, nullptr, nullptr, all);
-    if (!rc) rc = fft_backward_yx(c, zout_chi, c->chi, 1, all);
-    if (!rc && B->gr) rc = fft_backward_yx(c, zout_b, c->Bi, 3, all);
+    if (!rc) rc = launch_zsolve_tensor(c, c->SijFT, c->SijFT, 0., true, nullptr, nullptr, all);
+    // chi (component 0) and, in a GR run, B (components 1-3)
+    if (!rc) rc = fft_backward_yx(c, c->SijFT, c->chi, B->gr ? 4 : 1, all, c->Bi);
     return rc ? rc : check_hip(c, hipGetLastError(), "batch field stage");
 }
 

@@ -155,6 +155,101 @@ __device__ __forceinline__ void stages(C *lds, const C *tw) {
     }
 }
 
+// A tile of LINES interleaved columns of length L transformed with its first
+// and last stage working straight on registers: the first stage's operands
+// (element j + r L/R of column w) and the last stage's results (element
+// k + r NS) are whole rows of the tile, so they are loaded from and stored to
+// global memory in the butterflies' own layout and only the exchanges between
+// the stages go through LDS (2 instead of 4 round trips at L = 512).  The
+// arithmetic is that of stages().
+template <typename C, int L, int LINES, int NT> struct ColumnTile {
+    static constexpr int R1 = next_radix(L);           // first radix
+    static constexpr int M1 = L / R1;
+    static constexpr int JOBS1 = LINES * M1;
+    static constexpr int J1 = (JOBS1 + NT - 1) / NT;   // butterflies per thread
+    static constexpr bool SINGLE = R1 == L;            // one stage: no exchange at all
+
+    static_assert(NT % LINES == 0, "a thread keeps one column");
+
+    C v[J1][R1];
+
+    // Element e of this thread's column is ev() + eu with eu the same for
+    // every thread, so an address is one 32-bit offset per thread and a
+    // scalar base per element.
+    __device__ __forceinline__ static int column() { return threadIdx.x % LINES; }
+    __device__ __forceinline__ static int ev() { return threadIdx.x / LINES; }
+
+    // v = ld(eu) of this thread's first-stage butterflies
+    template <typename Ld> __device__ __forceinline__ void load(const Ld &ld) {
+#pragma unroll
+        for (int t = 0; t < J1; t++) {
+            const bool on = JOBS1 % NT == 0 || (int)threadIdx.x + t * NT < JOBS1;
+#pragma unroll
+            for (int r = 0; r < R1; r++) v[t][r] = on ? ld(t * (NT / LINES) + r * M1) : mk2<C>(0, 0);
+        }
+    }
+    template <bool CONJ> __device__ __forceinline__ static void conj_if(C (&x)[R1]) {
+        if (CONJ) {
+#pragma unroll
+            for (int r = 0; r < R1; r++) x[r] = cconj(x[r]);
+        }
+    }
+    // the first stage into LDS (of the conjugate if CONJ); v is free afterwards (the caller may start
+    // the next tile's loads) and the caller synchronises before finish()
+    template <bool CONJ> __device__ __forceinline__ void first(C *lds) {
+#pragma unroll
+        for (int t = 0; t < J1; t++) {
+            const int job = threadIdx.x + t * NT;
+            conj_if<CONJ>(v[t]);
+            Butterfly<C, R1>::run(v[t]);
+            if (JOBS1 % NT == 0 || job < JOBS1) {
+#pragma unroll
+                for (int r = 0; r < R1; r++) lds[(job / LINES * R1 + r) * LINES + job % LINES] = v[t][r];
+            }
+        }
+    }
+    // the remaining stages; st(eu, value) takes the results
+    template <int NS = R1, typename St>
+    __device__ __forceinline__ static void finish(C *lds, const C *tw, const St &st) {
+        constexpr int R = next_radix(L / NS);
+        static_assert(R == 2 || R == 3 || R == 4 || R == 8, "FFT length must be 2^a 3^b");
+        if constexpr (NS * R == L) {
+            constexpr int M = L / R, JOBS = LINES * M, J = (JOBS + NT - 1) / NT, TWS = L / (NS * R);
+#pragma unroll
+            for (int t = 0; t < J; t++) {
+                const int job = threadIdx.x + t * NT;
+                if (JOBS % NT == 0 || job < JOBS) {
+                    const int line = job % LINES, j = job / LINES;
+                    C x[R];
+#pragma unroll
+                    for (int r = 0; r < R; r++) x[r] = lds[(j + r * M) * LINES + line];
+#pragma unroll
+                    for (int r = 1; r < R; r++) x[r] = cmul(x[r], tw[j * r * TWS]);
+                    Butterfly<C, R>::run(x);
+#pragma unroll
+                    for (int r = 0; r < R; r++) st(t * (NT / LINES) + r * NS, x[r]);
+                }
+            }
+        } else {
+            stage<C, L, LINES, true, R, NS, NT>(lds, tw);
+            finish<NS * R>(lds, tw, st);
+        }
+    }
+    // results of a single-stage transform, straight from the registers
+    template <bool CONJ, typename St> __device__ __forceinline__ void finish_single(const St &st) {
+#pragma unroll
+        for (int t = 0; t < J1; t++) {
+            const int job = threadIdx.x + t * NT;
+            conj_if<CONJ>(v[t]);
+            Butterfly<C, R1>::run(v[t]);
+            if (JOBS1 % NT == 0 || job < JOBS1) {
+#pragma unroll
+                for (int r = 0; r < R1; r++) st(t * (NT / LINES) + r * M1, v[t][r]);
+            }
+        }
+    }
+};
+
 // lines of the x passes per workgroup: about 2048 complexes of LDS
 template <int N> constexpr int x_lines() {
     int m = N / 2, l = 1;
@@ -170,20 +265,26 @@ template <int N> constexpr int x_lines() {
 #ifndef GEV_COL_BYTES_F32
 #define GEV_COL_BYTES_F32 128
 #endif
-// threads per workgroup of the strided passes (FP64 / FP32 elements)
-#ifndef GEV_COL_TPB
-#define GEV_COL_TPB 256
-#endif
-#ifndef GEV_COL_TPB_F32
-#define GEV_COL_TPB_F32 512
-#endif
-template <typename T> constexpr int col_tpb() { return sizeof(T) == 4 ? GEV_COL_TPB_F32 : GEV_COL_TPB; }
 // RB: row bytes of a tile (0: the default of the form); the autotuner of a
 // batch may pick 64 or 256 instead
 template <typename T, int N, int RB = 0> constexpr int col_tile() {
     int w = (RB ? RB : (sizeof(T) == 4 ? GEV_COL_BYTES_F32 : GEV_COL_BYTES)) / (int)(2 * sizeof(T));
     while (w > 1 && w * N * (int)(2 * sizeof(T)) > 65536) w /= 2;
     return w;
+}
+// Threads per workgroup of the strided passes: one first-stage butterfly
+// each (a small tile takes a small workgroup, so more tiles share a CU), at
+// most GEV_COL_TPB / GEV_COL_TPB_F32 threads with several each.
+#ifndef GEV_COL_TPB
+#define GEV_COL_TPB 256
+#endif
+#ifndef GEV_COL_TPB_F32
+#define GEV_COL_TPB_F32 512
+#endif
+template <typename T, int N, int RB = 0> constexpr int col_tpb() {
+    constexpr int cap = sizeof(T) == 4 ? GEV_COL_TPB_F32 : GEV_COL_TPB;
+    constexpr int jobs = N / next_radix(N) * col_tile<T, N, RB>(), k = (jobs + cap - 1) / cap;
+    return ((jobs + k - 1) / k + 63) / 64 * 64;
 }
 
 }  // namespace gev_fft

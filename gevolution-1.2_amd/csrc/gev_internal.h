@@ -263,9 +263,11 @@ int fft_forward(gev_ctx *ctx, const double *real, double2 *kfield, int ncomp);
 int fft_backward(gev_ctx *ctx, const double2 *kfield, double *real, int ncomp);
 // the x and y passes only (the z pass fused with a solve follows), and the
 // backward transform of a field whose z pass is already done (in place on
-// kfield, which is scratch afterwards)
+// kfield, which is scratch afterwards; real_rest, when not null, takes the
+// components after the first)
 int fft_forward_xy(gev_ctx *ctx, const double *real, double2 *kfield, int ncomp, const Batch &bt = Batch{});
-int fft_backward_yx(gev_ctx *ctx, double2 *kfield, double *real, int ncomp, const Batch &bt = Batch{});
+int fft_backward_yx(gev_ctx *ctx, double2 *kfield, double *real, int ncomp, const Batch &bt = Batch{},
+                    double *real_rest = nullptr);
 // prepareFTsource fused into the first FFT pass (fftsolve.hip): Sij -> SijFT
 // and source (+ phi, chi) -> scalarFT, after the x pass only
 // A Batch with a BoxCycle array runs every box of the context's batch (box
