@@ -59,79 +59,179 @@ template <typename C> __device__ __forceinline__ double cross(const PkArgsT<C> &
     return p;
 }
 
+// A workgroup takes four rows at a time.  Each of its wavefronts forms one
+// row's terms in LDS and lists where the runs begin; then a lane sums one run
+// in kx order, run i of the four rows in neighbouring lanes, so the long runs
+// near kx = 0 (up to about 35 modes; 3 beyond) share a wavefront; then
+// wavefront q folds quantity q of the four rows into the histogram, row after
+// row.  The sums and their order are those of one mode after another.  Bound
+// by the instructions of the terms (FP64 roots and divisions) and of the
+// serial sums: with k_spectrum_reduce 1.33 ms at 512^3, 0.12 at 192^3, 26 us
+// at 64^3 (one row at a time per workgroup, and a serial column of loads per
+// thread in k_spectrum_reduce: 1.84, 0.38 and 0.23 ms).  Passing the sums
+// from lane to lane by shuffles took 3.2 ms at 512^3.
+// Occupations are whole numbers, added with LDS atomics in any order.
 template <int MAXH, typename C>
 __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
-    extern __shared__ double hist[];  // numbins * NQ
-    __shared__ int s_bin[MAXH];
-    __shared__ double s_q[NQ - 1][MAXH];
-    __shared__ int s_w[MAXH];
-    const int N = A.N, H = N / 2;
-    for (int t = threadIdx.x; t < A.numbins * NQ; t += TPB) hist[t] = 0.;
+    constexpr int WAVES = TPB / 64, J = (MAXH + 63) / 64;
+    static_assert(WAVES == NQ - 1, "a wavefront per summed quantity");
+    extern __shared__ double hist[];  // (NQ - 1) * numbins sums, then numbins counts (uint32)
+    __shared__ double s_tk[MAXH];                // typek2 of kx
+    __shared__ double s_q[3][WAVES][MAXH];       // weight * (k, P k^3 / s, (P k^3 / s)^2); a run's sum at its head
+    __shared__ double s_q1[WAVES][MAXH];         // a run's sum of weight * k^2 at its head
+    __shared__ int16_t s_bin[WAVES][MAXH];
+    __shared__ int16_t s_run[WAVES][MAXH + 1];   // where the runs begin (runs outside the bins too), and the end
+    __shared__ int s_n[WAVES];
+    uint32_t *const count = reinterpret_cast<uint32_t *>(hist + (NQ - 1) * A.numbins);
+    const int N = A.N, H = N / 2, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int t = threadIdx.x; t < A.numbins * (NQ - 1); t += TPB) hist[t] = 0.;
+    for (int t = threadIdx.x; t < A.numbins; t += TPB) count[t] = 0u;
+    for (int t = threadIdx.x; t <= H; t += TPB) s_tk[t] = A.typek2[t];
     const int64_t r0 = (int64_t)blockIdx.x * A.rows_per_block;
     const int64_t r1 = min(r0 + A.rows_per_block, (int64_t)N * N);
-    for (int64_t r = r0; r < r1; r++) {
-        const int ky = (int)(r % N), kz = (int)(r / N);
-        __syncthreads();  // previous row's runs are folded
-        for (int kx = threadIdx.x; kx <= H; kx += TPB) {
-            int bin = -1;
-            double q0 = 0., q1 = 0., q2 = 0., q3 = 0.;
-            int weight = 0;
-            if (!(kx == 0 && ky == 0 && kz == 0)) {
-                weight = (kx == 0 || (kx == N / 2 && N % 2 == 0)) ? 1 : 2;
-                const double k2 = A.typek2[kx] + A.typek2[ky] + A.typek2[kz];
-                double s = A.sinc[kx] * A.sinc[ky] * A.sinc[kz];
-                s *= s;
-                const double p = cross(A, r * A.P + kx);
-                const int i = (int)floor((double)((double)A.numbins * sqrt(k2 / A.k2max)));
-                if (i < A.numbins) {
-                    bin = i;
-                    q0 = weight * sqrt(k2);
-                    q1 = weight * k2;
-                    q2 = weight * p * k2 * sqrt(k2) / s;
-                    q3 = weight * p * p * k2 * k2 * k2 / s / s;
+    auto weight_of = [&](int kx) { return (kx == 0 || (kx == N / 2 && N % 2 == 0)) ? 1 : 2; };
+    for (int64_t rg = r0; rg < r1; rg += WAVES) {
+        __syncthreads();  // the tables are there, the previous rows are folded
+        const int64_t r = rg + wave;
+        int n = 0;  // runs of this row
+        if (r < r1) {
+            const int ky = (int)(r % N), kz = (int)(r / N);
+            const double tky = A.typek2[ky], tkz = A.typek2[kz], sky = A.sinc[ky], skz = A.sinc[kz];
+            int open = -2;  // the bin of the mode before these 64
+            for (int kb = 0; kb <= H; kb += 64) {
+                const int kx = kb + lane;
+                int bin = -1;
+                if (kx <= H) {
+                    double q0 = 0., q2 = 0., q3 = 0.;
+                    if (!(kx == 0 && ky == 0 && kz == 0)) {
+                        const int weight = weight_of(kx);
+                        const double k2 = s_tk[kx] + tky + tkz;
+                        double s = A.sinc[kx] * sky * skz;
+                        s *= s;
+                        const double p = cross(A, r * A.P + kx);
+                        const int i = (int)floor((double)((double)A.numbins * sqrt(k2 / A.k2max)));
+                        if (i < A.numbins) {
+                            bin = i;
+                            q0 = weight * sqrt(k2);
+                            q2 = weight * p * k2 * sqrt(k2) / s;
+                            q3 = weight * p * p * k2 * k2 * k2 / s / s;
+                        }
+                    }
+                    s_bin[wave][kx] = (int16_t)bin;
+                    s_q[0][wave][kx] = q0;
+                    s_q[1][wave][kx] = q2;
+                    s_q[2][wave][kx] = q3;
                 }
+                const int up = __shfl_up(bin, 1);
+                const bool head = kx <= H && bin != (lane == 0 ? open : up);
+                const uint64_t heads = __ballot(head);
+                if (head) s_run[wave][n + (int)__popcll(heads & ((1ull << lane) - 1ull))] = (int16_t)kx;
+                n += (int)__popcll(heads);
+                open = __shfl(bin, 63);
             }
-            s_bin[kx] = bin;
-            s_q[0][kx] = q0;
-            s_q[1][kx] = q1;
-            s_q[2][kx] = q2;
-            s_q[3][kx] = q3;
-            s_w[kx] = bin >= 0 ? weight : 0;
+            if (lane == 0) s_run[wave][n] = (int16_t)(H + 1);
+        }
+        if (lane == 0) s_n[wave] = n;
+        __syncthreads();
+        int most = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) most = max(most, s_n[w]);
+        for (int t = threadIdx.x; t < most * WAVES; t += TPB) {
+            const int w = t % WAVES, i = t / WAVES;
+            if (i >= s_n[w]) continue;
+            const int b = s_run[w][i], e = s_run[w][i + 1], bin = s_bin[w][b];
+            if (bin < 0) continue;
+            const int64_t row = rg + w;
+            const double tky = A.typek2[row % N], tkz = A.typek2[row / N];
+            double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
+            uint32_t m = 0;
+#pragma unroll 2
+            for (int k = b; k < e; k++) {
+                const int weight = weight_of(k);
+                const double k2 = s_tk[k] + tky + tkz;
+                a0 += s_q[0][w][k];
+                a1 += weight * k2;
+                a2 += s_q[1][w][k];
+                a3 += s_q[2][w][k];
+                m += weight;
+            }
+            // (a run's terms are read by this lane alone)
+            s_q[0][w][b] = a0;
+            s_q1[w][b] = a1;
+            s_q[1][w][b] = a2;
+            s_q[2][w][b] = a3;
+            atomicAdd(count + bin, m);
         }
         __syncthreads();
-        for (int kx = threadIdx.x; kx <= H; kx += TPB) {
-            const int bin = s_bin[kx];
-            if (bin < 0 || (kx > 0 && s_bin[kx - 1] == bin)) continue;  // not the head of a run
-            double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
-            int w = 0;
-            for (int j = kx; j <= H && s_bin[j] == bin; j++) {
-                a0 += s_q[0][j];
-                a1 += s_q[1][j];
-                a2 += s_q[2][j];
-                a3 += s_q[3][j];
-                w += s_w[j];
+        const double(*const src)[MAXH] = wave == 0 ? s_q[0] : wave == 1 ? s_q1 : wave == 2 ? s_q[1] : s_q[2];
+        double *const h = hist + wave * A.numbins;
+        for (int w = 0; w < WAVES; w++) {
+            // no two runs of a row share a bin: read, add and write them side by side
+            const int m = s_n[w];
+            int bin[J];
+            double v[J];
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                bin[j] = -1;
+                v[j] = 0.;
+                if (lane + 64 * j < m) {
+                    const int b = s_run[w][lane + 64 * j];
+                    bin[j] = s_bin[w][b];
+                    v[j] = src[w][b];
+                }
             }
-            double *h = hist + (int64_t)bin * NQ;
-            h[0] += a0;
-            h[1] += a1;
-            h[2] += a2;
-            h[3] += a3;
-            h[4] += (double)w;
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                if (bin[j] >= 0) v[j] = h[bin[j]] + v[j];
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                if (bin[j] >= 0) h[bin[j]] = v[j];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
     }
     __syncthreads();
     double *out = A.partial + (int64_t)blockIdx.x * A.numbins * NQ;
-    for (int t = threadIdx.x; t < A.numbins * NQ; t += TPB) out[t] = hist[t];
+    for (int t = threadIdx.x; t < A.numbins * NQ; t += TPB) {
+        const int bin = t / NQ, q = t % NQ;
+        out[t] = q < NQ - 1 ? hist[q * A.numbins + bin] : (double)count[bin];
+    }
 }
 
-// sums the workgroup histograms per bin, in workgroup order
+// Sums the workgroup histograms per bin, in workgroup order.  The sums are
+// serial by design (their order is fixed), the loads need not be: a workgroup
+// takes RED_COLS of the numbins * NQ sums, all its threads bring RED_ROWS
+// histograms into LDS while the previous ones are added (219 -> 11 us for
+// 1024 histograms of 32 bins, where each thread had loaded its own column).
+constexpr int RED_COLS = 16, RED_ROWS = 256, RED_PER = RED_ROWS * RED_COLS / TPB;
 __global__ __launch_bounds__(TPB) void k_spectrum_reduce(const double *__restrict__ partial, int nblk, int numbins,
                                                          double *__restrict__ total) {
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    if (t >= numbins * NQ) return;
+    __shared__ double s_p[RED_ROWS * RED_COLS];
+    const int ncol = numbins * NQ, cc = threadIdx.x % RED_COLS, rr = threadIdx.x / RED_COLS;
+    const int col = blockIdx.x * RED_COLS + cc;
+    double v[RED_PER];
+    auto load = [&](int b0) {
+#pragma unroll
+        for (int i = 0; i < RED_PER; i++) {
+            const int b = b0 + rr + i * (TPB / RED_COLS);
+            v[i] = b < nblk && col < ncol ? partial[(int64_t)b * ncol + col] : 0.;
+        }
+    };
+    load(0);
     double s = 0.;
-    for (int b = 0; b < nblk; b++) s += partial[(int64_t)b * numbins * NQ + t];
-    total[t] = s;
+    for (int b0 = 0; b0 < nblk; b0 += RED_ROWS) {
+#pragma unroll
+        for (int i = 0; i < RED_PER; i++) s_p[(rr + i * (TPB / RED_COLS)) * RED_COLS + cc] = v[i];
+        __syncthreads();
+        if (b0 + RED_ROWS < nblk) load(b0 + RED_ROWS);
+        if (rr == 0) {
+            const int m = min(RED_ROWS, nblk - b0);
+#pragma unroll 8
+            for (int b = 0; b < m; b++) s += s_p[b * RED_COLS + cc];
+        }
+        __syncthreads();
+    }
+    if (rr == 0 && col < ncol) total[col] = s;
 }
 
 }  // namespace
@@ -175,6 +275,14 @@ int64_t spectrum_scratch_doubles(int N, int numbins) {
     return 2 * (int64_t)N + ((int64_t)nblk + 1) * numbins * NQ;
 }
 
+// the row kernel with LDS for the rows of its grid size (more workgroups per CU on smaller grids)
+template <typename C> static void launch_rows(gev_ctx *c, const PkArgsT<C> &A, int nblk, size_t shm) {
+    const int h = c->N / 2 + 1;
+    if (h <= 65) hipLaunchKernelGGL((k_spectrum_rows<65, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+    else if (h <= 257) hipLaunchKernelGGL((k_spectrum_rows<257, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+    else hipLaunchKernelGGL((k_spectrum_rows<513, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+}
+
 // The spectrum with its device scratch given: the two tables (2N doubles),
 // the workgroup histograms and the bin totals, spectrum_scratch_doubles(N,
 // numbins) doubles in all.  tk, sn, tot: host buffers of N, N and numbins * NQ
@@ -209,7 +317,7 @@ static int spectrum_core(gev_ctx *c, const double2 *f1, const double2 *f2, int n
     A.partial = dpart;
     {
         ScopedTimer t(c, "power_spectrum");
-        const size_t shm = (size_t)numbins * NQ * 8;
+        const size_t shm = (size_t)numbins * ((NQ - 1) * 8 + 4);
         if (c->fp32) {
             // the same arguments over float2 fields
             PkArgsT<float2> B;
@@ -228,16 +336,11 @@ static int spectrum_core(gev_ctx *c, const double2 *f1, const double2 *f2, int n
             B.numbins = A.numbins;
             B.rows_per_block = A.rows_per_block;
             B.partial = A.partial;
-            if (N / 2 + 1 <= 257)
-                hipLaunchKernelGGL((k_spectrum_rows<257, float2>), dim3(nblk), dim3(TPB), shm, c->stream, B);
-            else
-                hipLaunchKernelGGL((k_spectrum_rows<513, float2>), dim3(nblk), dim3(TPB), shm, c->stream, B);
-        } else if (N / 2 + 1 <= 257) {
-            hipLaunchKernelGGL((k_spectrum_rows<257, double2>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+            launch_rows(c, B, nblk, shm);
         } else {
-            hipLaunchKernelGGL((k_spectrum_rows<513, double2>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+            launch_rows(c, A, nblk, shm);
         }
-        hipLaunchKernelGGL(k_spectrum_reduce, dim3((numbins * NQ + TPB - 1) / TPB), dim3(TPB), 0, c->stream,
+        hipLaunchKernelGGL(k_spectrum_reduce, dim3((numbins * NQ + RED_COLS - 1) / RED_COLS), dim3(TPB), 0, c->stream,
                            (const double *)dpart, nblk, numbins, dtot);
     }
     rc = check_hip(c, hipGetLastError(), "spectrum launch");
