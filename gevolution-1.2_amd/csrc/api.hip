@@ -703,9 +703,10 @@ static int cycle_fields(gev_ctx *c, const gev_sim_params *p, const gev_cycle_sta
     const gev_cosmology *cs = &p->cosmo;
     double a = st->a;
     int rc;
-    // phi(k=0) and chi(k=0) of the z solves (FP64): element 0 of scalarFT in
-    // the FP64 form, FP64 slots of the reduction scratch in the FP32 form
-    double2 *const phik0 = c->fp32 ? reinterpret_cast<double2 *>(c->red_d + 2) : c->scalarFT;
+    // the cycle's scalars in the reduction scratch: T00hom * N^3 in [1],
+    // phi(k=0) of the z solve in [2..3]; chi(k=0) in element 0 of scalarFT in
+    // the FP64 form, in an FP64 slot in the FP32 form
+    double2 *const phik0 = reinterpret_cast<double2 *>(c->red_d + 2);
     double2 *const chik0 = c->fp32 ? reinterpret_cast<double2 *>(c->red_d + 4) : c->scalarFT;
 
     // projection_init(source), projection_init(Sij) + T00 and Tij deposits
@@ -727,7 +728,7 @@ static int cycle_fields(gev_ctx *c, const gev_sim_params *p, const gev_cycle_sta
     }
 
     if (p->gr_flag > 0) {
-        rc = launch_field_sum(c, c->source, n3(c), nullptr);  // T00hom * N^3 -> red_d[0]
+        rc = launch_field_sum(c, c->source, n3(c), nullptr);  // T00hom * N^3 -> red_d[1]
         if (rc) return rc;
         if (st->dtau_old > 0.) {
             // prepareFTsource inside the first FFT pass, solveModifiedPoissonFT
@@ -749,16 +750,13 @@ static int cycle_fields(gev_ctx *c, const gev_sim_params *p, const gev_cycle_sta
         if (rc) return rc;
     }
     // phi(k=0) for the background record (main.cpp:533).  Without a solve in
-    // this cycle it is whatever scalarFT holds at k = 0 (widened in the FP32 form).
-    if (c->fp32 && p->gr_flag > 0 && !(st->dtau_old > 0.)) {
-        rc = launch_convert(c, c->scalarFT, true, phik0, false, 2);
+    // this cycle it is whatever scalarFT holds at k = 0.
+    if (p->gr_flag > 0 && !(st->dtau_old > 0.)) {
+        rc = launch_convert(c, c->scalarFT, c->fp32, phik0, false, 2);
         if (rc) return rc;
     }
-    rc = check_hip(c, hipMemcpyAsync(c->red_d + 1, phik0, sizeof(double),
-                                     hipMemcpyDeviceToDevice, c->stream), "phi_k0");
-    if (rc) return rc;
     if (rec) {
-        rc = check_hip(c, hipMemcpyAsync(rec, c->red_d, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream),
+        rc = check_hip(c, hipMemcpyAsync(rec, c->red_d + 1, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream),
                        "background record");
         if (rc) return rc;
     }
@@ -833,7 +831,7 @@ static int read_cycle_scalars(gev_ctx *c, const gev_sim_params *p, gev_cycle_sta
     double h[2];
     unsigned long long vb;
     int rc = check_hip(c, hipStreamSynchronize(c->stream), "cycle sync");
-    if (!rc) rc = check_hip(c, hipMemcpy(h, c->red_d, 2 * sizeof(double), hipMemcpyDeviceToHost), "cycle scalars");
+    if (!rc) rc = check_hip(c, hipMemcpy(h, c->red_d + 1, 2 * sizeof(double), hipMemcpyDeviceToHost), "cycle scalars");
     if (!rc) rc = check_hip(c, hipMemcpy(&vb, c->red_u, sizeof(vb), hipMemcpyDeviceToHost), "cycle vmax");
     if (rc) return rc;
     double mv;

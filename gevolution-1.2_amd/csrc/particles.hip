@@ -5,6 +5,7 @@
 //     listing each cell's particles in ascending ID.
 //   * updateVel / moveParticles with update_q(_Newton) / update_pos(_Newton)
 //     (gevolution.hpp:570-903), separately or fused into one particle pass.
+#include <algorithm>
 #include <utility>
 
 #include "gev_internal.h"
@@ -111,37 +112,55 @@ __global__ __launch_bounds__(TPB) void k_scan_reduce(const uint32_t *__restrict_
     }
 }
 
-// exclusive scan of the block partials in place (single workgroup)
+// exclusive scan of the block partials in place (single workgroup; the next
+// values are on their way while these are scanned: 65 -> 18 us at 512^3)
 __global__ __launch_bounds__(TPB) void k_scan_partials(uint32_t *__restrict__ part, int64_t nblk, gev::Batch bt) {
     if (!gev::box_on(bt, blockIdx.y)) return;
     part = gev::box_ptr(part, bt.stride, blockIdx.y);
-    const int64_t per = (nblk + TPB - 1) / TPB;
-    const int64_t b = (int64_t)threadIdx.x * per;
-    uint32_t s = 0;
-    for (int64_t k = 0; k < per; k++)
-        if (b + k < nblk) s += part[b + k];
-    uint32_t total;
-    uint32_t off = block_exclusive_scan(s, &total);
-    for (int64_t k = 0; k < per; k++)
-        if (b + k < nblk) {
-            uint32_t v = part[b + k];
-            part[b + k] = off;
-            off += v;
+    uint32_t carry = 0;
+    const int64_t i0 = 8 * (int64_t)threadIdx.x;
+    uint4 v = load4(part, i0, nblk), w = load4(part, i0 + 4, nblk);
+    for (int64_t base = 0; base < nblk; base += 8 * TPB) {
+        const uint4 x = v, y = w;
+        const int64_t i = base + i0;
+        v = load4(part, i + 8 * TPB, nblk);
+        w = load4(part, i + 8 * TPB + 4, nblk);
+        uint32_t total;
+        const uint32_t o[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        uint32_t off = carry + block_exclusive_scan(x.x + x.y + x.z + x.w + y.x + y.y + y.z + y.w, &total);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            if (i + k < nblk) part[i + k] = off;
+            off += o[k];
         }
+        carry += total;
+    }
 }
 
+// part: scanned partials, or (summed = false, few blocks) the plain ones,
+// which every block then adds up itself.  Also clears the sort's list counter.
 __global__ __launch_bounds__(TPB) void k_scan_final(const uint32_t *__restrict__ cnt, int64_t n,
-                                                    const uint32_t *__restrict__ part,
-                                                    uint32_t *__restrict__ out, gev::Batch bt) {
+                                                    const uint32_t *__restrict__ part, bool summed,
+                                                    uint32_t *__restrict__ out, uint32_t *__restrict__ nbig,
+                                                    gev::Batch bt) {
     if (!gev::box_on(bt, blockIdx.y)) return;
     cnt = gev::box_ptr(cnt, bt.stride, blockIdx.y);
     part = gev::box_ptr(part, bt.stride, blockIdx.y);
     out = gev::box_ptr(out, bt.stride, blockIdx.y);
+    nbig = gev::box_ptr(nbig, bt.stride, blockIdx.y);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nbig = 0u;
     const int64_t b0 = (int64_t)blockIdx.x * SCAN_BLOCK;
     uint4 v[SCAN_PASSES];
 #pragma unroll
     for (int k = 0; k < SCAN_PASSES; k++) v[k] = load4(cnt, b0 + 4 * ((int64_t)k * TPB + threadIdx.x), n);
-    uint32_t carry = part[blockIdx.x];
+    uint32_t carry;
+    if (summed) {
+        carry = part[blockIdx.x];
+    } else {
+        uint32_t s = 0;
+        for (uint32_t t = threadIdx.x; t < blockIdx.x; t += TPB) s += part[t];
+        (void)block_exclusive_scan(s, &carry);
+    }
 #pragma unroll
     for (int k = 0; k < SCAN_PASSES; k++) {
         const int64_t i = b0 + 4 * ((int64_t)k * TPB + threadIdx.x);
@@ -1222,8 +1241,7 @@ void launch_update_t(gev_ctx *ctx, const StepArgs &sa, const gev::Batch &bt = ge
 namespace gev {
 
 // scan count[] into start[] and build perm[] from cell[] (count[] ends zero).
-// Over a batch (bt.cyc set) every box is filed by the same launches; the
-// list counter sort_n of each box was cleared before the particle stage.
+// Over a batch (bt.cyc set) every box is filed by the same launches.
 static int finish_filing(gev_ctx *ctx, const Batch &bt = Batch{}) {
     const int64_t n3v = n3(ctx);
     const int64_t nblk = (n3v + SCAN_BLOCK - 1) / SCAN_BLOCK;
@@ -1232,9 +1250,13 @@ static int finish_filing(gev_ctx *ctx, const Batch &bt = Batch{}) {
         ScopedTimer t(ctx, "filing_scan");
         hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nblk, nb), dim3(TPB), 0, ctx->stream, ctx->count,
                            n3v, ctx->scan_part, bt);
-        hipLaunchKernelGGL(k_scan_partials, dim3(1, nb), dim3(TPB), 0, ctx->stream, ctx->scan_part, nblk, bt);
+        // up to 2048 blocks (192^3) add the partials before them up themselves:
+        // a launch less (12.6 -> 11.1 us for the scan at 64^3)
+        const bool scanned = nblk > 2048;
+        if (scanned)
+            hipLaunchKernelGGL(k_scan_partials, dim3(1, nb), dim3(TPB), 0, ctx->stream, ctx->scan_part, nblk, bt);
         hipLaunchKernelGGL(k_scan_final, dim3((unsigned)nblk, nb), dim3(TPB), 0, ctx->stream, ctx->count,
-                           n3v, ctx->scan_part, ctx->start, bt);
+                           n3v, ctx->scan_part, scanned, ctx->start, ctx->sort_n + 1, bt);
     }
     if (ctx->n > 0) {
         ScopedTimer t(ctx, "filing_scatter");
@@ -1243,29 +1265,29 @@ static int finish_filing(gev_ctx *ctx, const Batch &bt = Batch{}) {
     }
     {
         ScopedTimer t(ctx, "filing_sort");
-        // sort_n[1]: the number of listed cells
-        if (!bt.cyc) {
-            int rc = check_hip(ctx, hipMemsetAsync(ctx->sort_n, 0, 2 * sizeof(uint32_t), ctx->stream),
-                               "sort list clear");
-            if (rc) return rc;
-        }
         hipLaunchKernelGGL(k_sort_cells, dim3(grid_for(n3v, TPB), nb), dim3(TPB), 0, ctx->stream,
                            ctx->start, ctx->id, n3v, ctx->perm, reinterpret_cast<uint8_t *>(ctx->sort_segs), ctx->id2,
                            bt);
     }
     {
         ScopedTimer t(ctx, "filing_sort_segments");
-        // SORT_SEG_BATCH segments per workgroup: the late, clustered cycles flag
-        // most segments and need the parallelism; early ones flag almost none
-        const unsigned nsw = (unsigned)((grid_for(n3v, TPB) + SORT_SEG_BATCH - 1) / SORT_SEG_BATCH);
+        // Up to SORT_SEG_BATCH segments per workgroup: the late, clustered cycles
+        // flag most segments and need the parallelism; early ones flag almost
+        // none.  Small grids (their boxes together) spread their segments over
+        // the chip instead: 156 -> 22 us at 64^3, z = 1 (it was 32 workgroups
+        // of 32 segments), 43 -> 13 us at 128^3, z = 10; 256^3 has 2048
+        // workgroups either way (4096 were slower: 256 against 242 us).
+        const unsigned nseg = grid_for(n3v, TPB), full = std::max(1u, 2048u / nb);
+        const unsigned nsw = std::max((nseg + SORT_SEG_BATCH - 1) / SORT_SEG_BATCH, std::min(nseg, full));
         hipLaunchKernelGGL(k_sort_segments, dim3(nsw, nb), dim3(TPB), 0, ctx->stream, ctx->start, ctx->id, n3v,
                            ctx->perm, reinterpret_cast<const uint8_t *>(ctx->sort_segs),
                            (uint32_t)grid_for(n3v, TPB), ctx->sort_big, ctx->sort_n + 1, ctx->id2, bt);
     }
     {
         ScopedTimer t(ctx, "filing_sort_dense_cells");
-        hipLaunchKernelGGL(k_sort_big, dim3(1024, nb), dim3(TPB), 0, ctx->stream, ctx->start, ctx->id, ctx->perm,
-                           ctx->sort_big, ctx->sort_n + 1, ctx->id2, bt);
+        // (1024 workgroups in all, at least 32 per box: 48 boxes of 32^3 had 49152)
+        hipLaunchKernelGGL(k_sort_big, dim3(std::max(1024u / nb, 32u), nb), dim3(TPB), 0, ctx->stream, ctx->start,
+                           ctx->id, ctx->perm, ctx->sort_big, ctx->sort_n + 1, ctx->id2, bt);
     }
     const int rc = check_hip(ctx, hipGetLastError(), "filing launch");
     if (!rc) ctx->count_clean = true;  // the scatter counted every cell back to zero

@@ -131,7 +131,7 @@ int launch_prepare_tensor(gev_ctx *ctx, double coeff) {
 }
 
 // sums count field elements (double, or float in the FP32 form) into
-// ctx->red_d[0] in FP64; copies to *out_host if non-null (sync)
+// ctx->red_d[1] in FP64; copies to *out_host if non-null (sync)
 int launch_field_sum(gev_ctx *ctx, const double *f, int64_t count, double *out_host) {
     const int64_t per = (int64_t)TPB * SUM_ITEMS;
     const int64_t nblk = (count + per - 1) / per;
@@ -145,12 +145,12 @@ int launch_field_sum(gev_ctx *ctx, const double *f, int64_t count, double *out_h
             hipLaunchKernelGGL(k_sum_partial<double>, dim3((unsigned)nblk), dim3(TPB), 0, ctx->stream, f, count,
                                ctx->red_d + 8);
         hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(TPB), 0, ctx->stream, ctx->red_d + 8, nblk,
-                           ctx->red_d);
+                           ctx->red_d + 1);
     }
     int rc = check_hip(ctx, hipGetLastError(), "field sum launch");
     if (rc) return rc;
     if (out_host) {
-        rc = check_hip(ctx, hipMemcpyAsync(ctx->host_pinned, ctx->red_d, sizeof(double),
+        rc = check_hip(ctx, hipMemcpyAsync(ctx->host_pinned, ctx->red_d + 1, sizeof(double),
                                            hipMemcpyDeviceToHost, ctx->stream),
                        "field sum readback");
         if (rc) return rc;
