@@ -347,6 +347,11 @@ template <typename F, typename C> struct XArgsT {
 };
 using XArgs = XArgsT<double, double2>;
 
+// NC: 1 the scalar source, 6 the tensor's components in one workgroup (phi
+// is read once for all), TENSOR_ONE the tensor with one component per
+// workgroup (blockIdx.z), for grids whose rows would not fill the chip.
+constexpr int TENSOR_ONE = -6;
+
 // Rows per workgroup: the NC prepared components of a thread's points are
 // held in registers until each is transformed, so the 6-component form
 // takes at most GEV_XPREP_PTS points per thread and component.
@@ -355,6 +360,7 @@ using XArgs = XArgsT<double, double2>;
 #endif
 template <int N, int NC> constexpr int xprep_lines() {
     int l = x_lines<N>();
+    while (NC == TENSOR_ONE && l > 1 && l * (N / 2) > 512) l /= 2;
     while (NC > 1 && l > 1 && l * (N / 2) > GEV_XPREP_PTS * 256) l /= 2;
     return l;
 }
@@ -363,6 +369,7 @@ template <int N, int NC, typename F, typename C>
 __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
     using R = decltype(C::x);
     constexpr int TPB = 256;
+    constexpr int NV = NC == 6 ? 6 : 1;  // components of this workgroup
     constexpr int M = N / 2;
     constexpr int LINES = xprep_lines<N, NC>();
     constexpr int PER = (LINES * M + TPB - 1) / TPB;
@@ -377,7 +384,7 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
         A.chi = gev::box_ptr(A.chi, A.bt.stride, b);
         A.src = gev::box_ptr(A.src, A.bt.stride, b);
         A.out = gev::box_ptr(A.out, A.bt.stride, b);
-        if (NC == 6) {
+        if (NC != 1) {
             A.c0 = bc.tens_c;
         } else {
             A.c0 = bc.prep_bg;
@@ -386,16 +393,20 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
             A.c3 = bc.prep_c3;
         }
     }
+    if (NC == TENSOR_ONE) {
+        A.src += blockIdx.z * A.n3v;
+        A.out += blockIdx.z * A.nkv;
+    }
     const int64_t row0 = (int64_t)blockIdx.x * LINES;
     for (int t = threadIdx.x; t < M; t += TPB) tw[t] = A.tw[2 * t];
-    C v[NC][PER];
+    C v[NV][PER];
 #pragma unroll
     for (int k = 0; k < PER; k++) {
         const int idx = threadIdx.x + k * TPB;
         const int line = idx / M, n = idx % M;
         const int64_t row = row0 + line;
 #pragma unroll
-        for (int c = 0; c < NC; c++) v[c][k] = mk2<C>(0, 0);
+        for (int c = 0; c < NV; c++) v[c][k] = mk2<C>(0, 0);
         if (!((EXACT || idx < LINES * M) && row < A.nrows)) continue;
         const int y = (int)(row % N), z = (int)(row / N);
 #pragma unroll
@@ -403,26 +414,20 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
             const int x = 2 * n + h;
             const int64_t i = row * N + x;
             const Nb c = nb_of(x, y, z, N);
-            if constexpr (NC == 6 && is_f32<C>()) {
-                float T[6], S[6];
+            if constexpr (NC == 6) {
+                F T[6], S[6];
 #pragma unroll
                 for (int q = 0; q < 6; q++) T[q] = A.src[q * A.n3v + i];
-                prep_tensor_f32(A.phi, T, c, i, N, (float)A.c0, S);
+                prep_tensor(A.phi, T, c, i, N, (F)A.c0, S);
 #pragma unroll
                 for (int q = 0; q < 6; q++) {
                     if (h == 0) v[q][k].x = S[q];
                     else v[q][k].y = S[q];
                 }
-            } else if constexpr (NC == 6) {
-                double T[6], S[6];
-#pragma unroll
-                for (int q = 0; q < 6; q++) T[q] = A.src[q * A.n3v + i];
-                prep_tensor(A.phi, T, c, i, N, A.c0, S);
-#pragma unroll
-                for (int q = 0; q < 6; q++) {
-                    if (h == 0) v[q][k].x = (R)S[q];
-                    else v[q][k].y = (R)S[q];
-                }
+            } else if constexpr (NC == TENSOR_ONE) {
+                const F r = prep_tensor_one(A.phi, A.src[i], c, i, N, (F)A.c0, (int)blockIdx.z);
+                if (h == 0) v[0][k].x = r;
+                else v[0][k].y = r;
             } else {
                 const double r = prep_scalar(A.phi, (double)A.chi[i], (double)A.src[i], c, i, N, A.c0, A.c1, A.c2, A.c3);
                 if (h == 0) v[0][k].x = (R)r;
@@ -431,7 +436,7 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
         }
     }
 #pragma unroll
-    for (int q = 0; q < NC; q++) {
+    for (int q = 0; q < NV; q++) {
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const int idx = threadIdx.x + k * TPB;
@@ -457,6 +462,17 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
 template <int N, int NC, typename F, typename C> int launch_x(gev_ctx *c, const XArgsT<F, C> &A) {
     constexpr int LINES = xprep_lines<N, NC>();
     const unsigned nbox = A.bt.cyc ? (unsigned)c->nbox : 1u;
+    // A tensor pass of fewer workgroups than two per CU takes one component in
+    // each instead, which re-reads phi from L2 (64^3: 15.9 -> 11.8 us, 32^3:
+    // 13.4 -> 7.4; 96^3, 576 workgroups: equal; 128^3, 1024: 61 -> 80)
+    if constexpr (NC == 6 && N <= 128) {
+        constexpr int L1 = xprep_lines<N, TENSOR_ONE>();
+        if (gev::grid_for(A.nrows, LINES) * nbox < 512) {
+            hipLaunchKernelGGL((k_r2c_x_prep<N, TENSOR_ONE, F, C>), dim3(gev::grid_for(A.nrows, L1), nbox, 6), dim3(256),
+                               0, c->stream, A);
+            return gev::check_hip(c, hipGetLastError(), "fused x pass launch");
+        }
+    }
     hipLaunchKernelGGL((k_r2c_x_prep<N, NC, F, C>), dim3(gev::grid_for(A.nrows, LINES), nbox), dim3(256), 0,
                        c->stream, A);
     return gev::check_hip(c, hipGetLastError(), "fused x pass launch");

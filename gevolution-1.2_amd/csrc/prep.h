@@ -51,69 +51,68 @@ __device__ __forceinline__ double prep_scalar(const F *__restrict__ phi, double 
     return r;
 }
 
-// prepareFTsource (1), gevolution.hpp:56-147: S[6] (order 00,01,02,11,12,22)
-// from the deposited T[6] at site i
-template <typename F>
-__device__ __forceinline__ void prep_tensor(const F *__restrict__ phi, const double T[6], const Nb &c,
-                                            int64_t i, int N, double coeff, double S[6]) {
-    const double p = phi[i];
-    const double px = phi[L(N, c.xp, c.y, c.z)], mx = phi[L(N, c.xm, c.y, c.z)];
-    const double py = phi[L(N, c.x, c.yp, c.z)], my = phi[L(N, c.x, c.ym, c.z)];
-    const double pz = phi[L(N, c.x, c.y, c.zp)], mz = phi[L(N, c.x, c.y, c.zm)];
-    const double pxy = phi[L(N, c.xp, c.yp, c.z)];
-    const double pxz = phi[L(N, c.xp, c.y, c.zp)];
-    const double pyz = phi[L(N, c.x, c.yp, c.zp)];
-    double s;
-    s = coeff * T[0];
-    s += 0.5 * (px - mx) * (px - mx);
-    S[0] = s;
-    s = coeff * T[3];
-    s += 0.5 * (py - my) * (py - my);
-    S[3] = s;
-    s = coeff * T[5];
-    s += 0.5 * (pz - mz) * (pz - mz);
-    S[5] = s;
-    s = coeff * T[1];
-    s += px * py - p * pxy;
+// The terms of prepareFTsource (1), gevolution.hpp:56-147, of one component
+// with the deposited value t: i = j from phi above and below along i, i != j
+// from phi on the plaquette's corners.
+__device__ __forceinline__ double prep_diag(double t, double up, double dn, double coeff) {
+    double s = coeff * t;
+    s += 0.5 * (up - dn) * (up - dn);
+    return s;
+}
+__device__ __forceinline__ double prep_off(double t, double p, double pa, double pb, double pab, double coeff) {
+    double s = coeff * t;
+    s += pa * pb - p * pab;
     s += 0.5 * p * p;
-    s -= 0.5 * px * px;
-    s -= 0.5 * py * py;
-    s += 0.5 * pxy * pxy;
-    S[1] = s;
-    s = coeff * T[2];
-    s += px * pz - p * pxz;
-    s += 0.5 * p * p;
-    s -= 0.5 * px * px;
-    s -= 0.5 * pz * pz;
-    s += 0.5 * pxz * pxz;
-    S[2] = s;
-    s = coeff * T[4];
-    s += py * pz - p * pyz;
-    s += 0.5 * p * p;
-    s -= 0.5 * py * py;
-    s -= 0.5 * pz * pz;
-    s += 0.5 * pyz * pyz;
-    S[4] = s;
+    s -= 0.5 * pa * pa;
+    s -= 0.5 * pb * pb;
+    s += 0.5 * pab * pab;
+    return s;
+}
+// ... in the FP32 form: the same terms over the float fields, evaluated in float
+__device__ __forceinline__ float prep_diag(float t, float up, float dn, float coeff) {
+    return coeff * t + 0.5f * (up - dn) * (up - dn);
+}
+__device__ __forceinline__ float prep_off(float t, float p, float pa, float pb, float pab, float coeff) {
+    const float hp = 0.5f * p * p, ha = 0.5f * pa * pa, hb = 0.5f * pb * pb;
+    return coeff * t + (pa * pb - p * pab) + hp - ha - hb + 0.5f * pab * pab;
 }
 
-// prepareFTsource (1) in the FP32 form: the same terms as prep_tensor over the
-// float fields, evaluated in float
-__device__ __forceinline__ void prep_tensor_f32(const float *__restrict__ phi, const float T[6], const Nb &c,
-                                                int64_t i, int N, float coeff, float S[6]) {
-    const float p = phi[i];
-    const float px = phi[L(N, c.xp, c.y, c.z)], mx = phi[L(N, c.xm, c.y, c.z)];
-    const float py = phi[L(N, c.x, c.yp, c.z)], my = phi[L(N, c.x, c.ym, c.z)];
-    const float pz = phi[L(N, c.x, c.y, c.zp)], mz = phi[L(N, c.x, c.y, c.zm)];
-    const float pxy = phi[L(N, c.xp, c.yp, c.z)];
-    const float pxz = phi[L(N, c.xp, c.y, c.zp)];
-    const float pyz = phi[L(N, c.x, c.yp, c.zp)];
-    const float hp = 0.5f * p * p, hx = 0.5f * px * px, hy = 0.5f * py * py, hz = 0.5f * pz * pz;
-    S[0] = coeff * T[0] + 0.5f * (px - mx) * (px - mx);
-    S[3] = coeff * T[3] + 0.5f * (py - my) * (py - my);
-    S[5] = coeff * T[5] + 0.5f * (pz - mz) * (pz - mz);
-    S[1] = coeff * T[1] + (px * py - p * pxy) + hp - hx - hy + 0.5f * pxy * pxy;
-    S[2] = coeff * T[2] + (px * pz - p * pxz) + hp - hx - hz + 0.5f * pxz * pxz;
-    S[4] = coeff * T[4] + (py * pz - p * pyz) + hp - hy - hz + 0.5f * pyz * pyz;
+// S[6] (order 00,01,02,11,12,22) from the deposited T[6] at site i (F: the
+// field element, and the type the stencils are evaluated in)
+template <typename F>
+__device__ __forceinline__ void prep_tensor(const F *__restrict__ phi, const F T[6], const Nb &c, int64_t i, int N,
+                                            F coeff, F S[6]) {
+    const F p = phi[i];
+    const F px = phi[L(N, c.xp, c.y, c.z)], mx = phi[L(N, c.xm, c.y, c.z)];
+    const F py = phi[L(N, c.x, c.yp, c.z)], my = phi[L(N, c.x, c.ym, c.z)];
+    const F pz = phi[L(N, c.x, c.y, c.zp)], mz = phi[L(N, c.x, c.y, c.zm)];
+    const F pxy = phi[L(N, c.xp, c.yp, c.z)];
+    const F pxz = phi[L(N, c.xp, c.y, c.zp)];
+    const F pyz = phi[L(N, c.x, c.yp, c.zp)];
+    S[0] = prep_diag(T[0], px, mx, coeff);
+    S[3] = prep_diag(T[3], py, my, coeff);
+    S[5] = prep_diag(T[5], pz, mz, coeff);
+    S[1] = prep_off(T[1], p, px, py, pxy, coeff);
+    S[2] = prep_off(T[2], p, px, pz, pxz, coeff);
+    S[4] = prep_off(T[4], p, py, pz, pyz, coeff);
+}
+
+// one component of it (q in the order above, the same for a whole wavefront)
+template <typename F>
+__device__ __forceinline__ F prep_tensor_one(const F *__restrict__ phi, F t, const Nb &c, int64_t i, int N, F coeff,
+                                             int q) {
+    const F p = phi[i];
+    switch (q) {
+    case 0: return prep_diag(t, phi[L(N, c.xp, c.y, c.z)], phi[L(N, c.xm, c.y, c.z)], coeff);
+    case 3: return prep_diag(t, phi[L(N, c.x, c.yp, c.z)], phi[L(N, c.x, c.ym, c.z)], coeff);
+    case 5: return prep_diag(t, phi[L(N, c.x, c.y, c.zp)], phi[L(N, c.x, c.y, c.zm)], coeff);
+    case 1:
+        return prep_off(t, p, phi[L(N, c.xp, c.y, c.z)], phi[L(N, c.x, c.yp, c.z)], phi[L(N, c.xp, c.yp, c.z)], coeff);
+    case 2:
+        return prep_off(t, p, phi[L(N, c.xp, c.y, c.z)], phi[L(N, c.x, c.y, c.zp)], phi[L(N, c.xp, c.y, c.zp)], coeff);
+    default:
+        return prep_off(t, p, phi[L(N, c.x, c.yp, c.z)], phi[L(N, c.x, c.y, c.zp)], phi[L(N, c.x, c.yp, c.zp)], coeff);
+    }
 }
 
 }  // namespace gev_prep
