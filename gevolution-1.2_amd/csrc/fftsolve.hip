@@ -117,6 +117,86 @@ template <typename C> struct ZArgsT {
 };
 using ZArgs = ZArgsT<double2>;
 
+// the k tables of a column
+struct KRow {
+    double gx, gy;
+    double2 kxs, kys;
+};
+template <typename C> __device__ __forceinline__ KRow k_row(const ZArgsT<C> &A, int kx, int ky, bool ok) {
+    return KRow{A.g[ok ? kx : 0], A.g[ky], A.ks[ok ? kx : 0], A.ks[ky]};
+}
+
+// The solve of one k point (kx, ky, kz) from its transformed inputs S, in
+// FP64 (the FP32 form's tensor solves: FP64 coefficients and denominators,
+// float field combinations); the outputs O are kept in the storage type (k = 0
+// of output 0 also in FP64).  at: the point's index in a k field.  HAVE_B: Bo
+// holds the carried B of the point, otherwise it is read here.
+template <int N, int KIND, bool HAVE_B, typename C>
+__device__ __forceinline__ void solve_point(const ZArgsT<C> &A, const KRow &row, int kx, int ky, int kz, bool live,
+                                            int64_t at, const C *S, const C *Bo, C *O) {
+    const double gx = row.gx, gy = row.gy, gz = A.g[live ? kz : 0];
+    const double2 kxs = row.kxs, kys = row.kys, kzs = A.ks[live ? kz : 0];
+    const bool zero = kx == 0 && ky == 0 && kz == 0;
+    auto carried = [&](int c) { return HAVE_B ? Bo[c] : A.bift[c * A.nkv + at]; };
+    double2 o0;
+    if constexpr (KIND == ZS_POISSON) {
+        o0 = poisson_point(d2(S[0]), zero, zero ? 0. : gx + gy + gz, A.c0, A.c1);
+    } else if constexpr ((KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) && is_f32<C>()) {
+        const float2 chi = zero ? make_float2(0.f, 0.f) : project_scalar_f32(S, gx, gy, gz, kxs, kys, kzs, N);
+        o0 = make_double2(chi.x, chi.y);
+        if constexpr (KIND == ZS_TENSOR) {
+            float2 B[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+            if (live) {
+                if (!zero) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) B[c] = carried(c);
+                    evolve_vector_f32(S, B, gx, gy, gz, kxs, kys, kzs, A.c0);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = B[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) O[1 + c] = B[c];
+        }
+    } else if constexpr (KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) {
+        double2 Sp[6];
+#pragma unroll
+        for (int c = 0; c < 6; c++) Sp[c] = d2(S[c]);
+        o0 = zero ? c2(0., 0.) : project_scalar(Sp, gx, gy, gz, kxs, kys, kzs, N);
+        if constexpr (KIND == ZS_TENSOR) {
+            double2 B[3] = {c2(0., 0.), c2(0., 0.), c2(0., 0.)};
+            if (live) {
+                if (!zero) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) B[c] = d2(carried(c));
+                    evolve_vector(Sp, B, gx, gy, gz, kxs, kys, kzs, A.c0);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = from_d2<C>(B[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) O[1 + c] = from_d2<C>(B[c]);
+        }
+    } else {
+        double2 Sv[3] = {d2(S[0]), d2(S[1]), d2(S[2])};
+        if (zero) {
+            Sv[0] = Sv[1] = Sv[2] = c2(0., 0.);
+        } else {
+            project_vector_point(Sv, kxs, kys, kzs, gx + gy + gz, A.c0, A.c1);
+        }
+        if (live && A.bift) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = from_d2<C>(Sv[c]);
+        }
+        o0 = Sv[0];
+#pragma unroll
+        for (int c = 1; c < 3; c++) O[c] = from_d2<C>(Sv[c]);
+    }
+    O[0] = from_d2<C>(o0);
+    if (live && A.kstore) A.kstore[at] = O[0];
+    if (zero && A.k0) A.k0[0] = o0;
+}
+
 template <int N, int KIND, typename C>
 __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C> A) {
     constexpr int W = zs_cols<N, KIND, C>();
@@ -214,100 +294,25 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
         }
     }
 
-    // the solve, per k point (kx, ky, kz = element index), in FP64; the
-    // outputs are kept in the storage type (k = 0 of output 0 also in FP64)
+    // the solve, per k point (kx, ky, kz = element index)
     C O[NOUT][PTS];
-    const double gx = A.g[ok ? kx : 0];
-    const double2 kxs = A.ks[ok ? kx : 0];
-    const double gy = A.g[ky];
-    const double2 kys = A.ks[ky];
+    const KRow row = k_row(A, kx, ky, ok);
 #pragma unroll
     for (int j = 0; j < PTS; j++) {
         const int idx = threadIdx.x + j * NT;
         const int kz = idx / W;
         const bool live = ok && (EXACT || idx < N * W);
-        const double gz = A.g[live ? kz : 0];
-        const double2 kzs = A.ks[live ? kz : 0];
-        const bool zero = kx == 0 && ky == 0 && kz == 0;
-        const int64_t at = base + (int64_t)kz * es + w;
-        double2 o0;
-        if constexpr (KIND == ZS_POISSON) {
-            o0 = poisson_point(d2(S[0][j]), zero, zero ? 0. : gx + gy + gz, A.c0, A.c1);
-        } else if constexpr ((KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) && is_f32<C>()) {
-            // FP32 form: FP64 coefficients and denominators, float field combinations
-            float2 Sf[6];
+        C Sj[NIN], Oj[NOUT], Bj[3];
 #pragma unroll
-            for (int c = 0; c < 6; c++) Sf[c] = S[c][j];
-            const float2 chi = zero ? make_float2(0.f, 0.f) : project_scalar_f32(Sf, gx, gy, gz, kxs, kys, kzs, N);
-            o0 = make_double2(chi.x, chi.y);
-            if constexpr (KIND == ZS_TENSOR) {
-                float2 B[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-                if (live) {
-                    if (!zero) {
-                        if constexpr (zs_prefetch_b<N, C>()) {
-                            B[0] = Bold[0][j];
-                            B[1] = Bold[KIND == ZS_TENSOR ? 1 : 0][j];
-                            B[2] = Bold[KIND == ZS_TENSOR ? 2 : 0][j];
-                        } else {
-                            B[0] = A.bift[at];
-                            B[1] = A.bift[A.nkv + at];
-                            B[2] = A.bift[2 * A.nkv + at];
-                        }
-                        evolve_vector_f32(Sf, B, gx, gy, gz, kxs, kys, kzs, A.c0);
-                    }
-                    A.bift[at] = B[0];
-                    A.bift[A.nkv + at] = B[1];
-                    A.bift[2 * A.nkv + at] = B[2];
-                }
+        for (int c = 0; c < NIN; c++) Sj[c] = S[c][j];
+        if constexpr (KIND == ZS_TENSOR && zs_prefetch_b<N, C>()) {
 #pragma unroll
-                for (int c = 0; c < 3; c++) O[1 + c][j] = B[c];
-            }
-        } else if constexpr (KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) {
-            double2 Sp[6];
-#pragma unroll
-            for (int c = 0; c < 6; c++) Sp[c] = d2(S[c][j]);
-            o0 = zero ? c2(0., 0.) : project_scalar(Sp, gx, gy, gz, kxs, kys, kzs, N);
-            if constexpr (KIND == ZS_TENSOR) {
-                double2 B[3] = {c2(0., 0.), c2(0., 0.), c2(0., 0.)};
-                if (live) {
-                    if (!zero) {
-                        if constexpr (zs_prefetch_b<N, C>()) {
-                            B[0] = d2(Bold[0][j]);
-                            B[1] = d2(Bold[KIND == ZS_TENSOR ? 1 : 0][j]);
-                            B[2] = d2(Bold[KIND == ZS_TENSOR ? 2 : 0][j]);
-                        } else {
-                            B[0] = d2(A.bift[at]);
-                            B[1] = d2(A.bift[A.nkv + at]);
-                            B[2] = d2(A.bift[2 * A.nkv + at]);
-                        }
-                        evolve_vector(Sp, B, gx, gy, gz, kxs, kys, kzs, A.c0);
-                    }
-                    A.bift[at] = from_d2<C>(B[0]);
-                    A.bift[A.nkv + at] = from_d2<C>(B[1]);
-                    A.bift[2 * A.nkv + at] = from_d2<C>(B[2]);
-                }
-#pragma unroll
-                for (int c = 0; c < 3; c++) O[1 + c][j] = from_d2<C>(B[c]);
-            }
-        } else {
-            double2 Sv[3] = {d2(S[0][j]), d2(S[1][j]), d2(S[2][j])};
-            if (zero) {
-                Sv[0] = Sv[1] = Sv[2] = c2(0., 0.);
-            } else {
-                project_vector_point(Sv, kxs, kys, kzs, gx + gy + gz, A.c0, A.c1);
-            }
-            if (live && A.bift) {
-                A.bift[at] = from_d2<C>(Sv[0]);
-                A.bift[A.nkv + at] = from_d2<C>(Sv[1]);
-                A.bift[2 * A.nkv + at] = from_d2<C>(Sv[2]);
-            }
-            o0 = Sv[0];
-#pragma unroll
-            for (int c = 1; c < 3; c++) O[c][j] = from_d2<C>(Sv[c]);
+            for (int c = 0; c < 3; c++) Bj[c] = Bold[c][j];
         }
-        O[0][j] = from_d2<C>(o0);
-        if (live && A.kstore) A.kstore[at] = O[0][j];
-        if (zero && A.k0) A.k0[0] = o0;
+        solve_point<N, KIND, (KIND == ZS_TENSOR && zs_prefetch_b<N, C>())>(A, row, kx, ky, kz, live,
+                                                                           base + (int64_t)kz * es + w, Sj, Bj, Oj);
+#pragma unroll
+        for (int o = 0; o < NOUT; o++) O[o][j] = Oj[o];
     }
 
     // inverse z transform of every output (conjugate, forward stages, conjugate)
@@ -325,6 +330,194 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
             const int idx = threadIdx.x + j * NT;
             if (ok && (EXACT || idx < N * W))
                 A.out[o * A.nkv + base + (int64_t)(idx / W) * es + w] = cconj(buf[idx]);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- direct form
+//
+// The FP64 tensor solve with the carried B, for powers of two from 64.  A
+// transform's first stage reads, and its last stage leaves, 8 points of a
+// column per thread: kz = ev + m N / 8 (m < 8, ev = its butterfly).  The loads,
+// the solve, the inverse transform's first stage and the stores work on these
+// registers, and LDS carries only the exchanges between stages (2 round trips
+// per transform at N = 512 where k_zsolve makes 4).  6 components x 8 points
+// do not fit the registers of a thread: the workgroup is two groups of threads
+// that transform two components at once and trade halves through LDS, so that
+// each thread solves 4 points of all components; half as many barriers as
+// k_zsolve, and two components' loads in flight.
+// Bound by the latency of its loads and barriers at 8 waves per CU (the
+// registers; 3 TB/s at 512^3).  us per launch, k_zsolve -> this: 512^3 4756 ->
+// 4640, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.7 -> 17.4, 32^3 12.1
+// both.  FP32 stays on k_zsolve: its float points leave a thread room for 8
+// points of all components only with spills (512^3 3012 -> 3432, 256^3 344 ->
+// 572); so do the FP64 solves with fewer fields (Poisson 512^3 620 -> 636, chi
+// alone 256^3 294 -> 305).
+template <int N, int KIND, typename C> constexpr bool zd_direct() {
+    return !is_f32<C>() && KIND == ZS_TENSOR && N >= 64 && (N & (N - 1)) == 0;
+}
+// columns per workgroup: 64-byte rows where the two buffers and the traded
+// halves fit LDS
+template <int N> constexpr int zd_cols() { return N >= 1024 ? 2 : 4; }
+template <int N> constexpr int zd_threads() { return 2 * N * zd_cols<N>() / 8; }
+
+// The transform of 8 points per thread (column w, points ev + m N / 8) of
+// N x W points in LDS; then() runs once the inputs are in LDS.  The caller
+// synchronises between transforms that use the same buf.
+template <typename C, int N, int W, int NS, int R>
+__device__ __forceinline__ void zd_read(C (&x)[8], const C *buf, const C *tw, int ev, int w) {
+    constexpr int J = 8 / R, TWS = N / (NS * R);
+#pragma unroll
+    for (int t = 0; t < J; t++) {
+        const int j = ev + t * (N / 8), k = j % NS;
+        C *const u = x + t * R;
+#pragma unroll
+        for (int r = 0; r < R; r++) u[r] = buf[(j + r * (N / R)) * W + w];
+#pragma unroll
+        for (int r = 1; r < R; r++) u[r] = cmul(u[r], tw[k * r * TWS]);
+        Butterfly<C, R>::run(u);
+    }
+}
+template <typename C, int N, int W, int NS>
+__device__ __forceinline__ void zd_stages(C (&out)[8], C *buf, const C *tw, int ev, int w) {
+    constexpr int R = next_radix(N / NS), J = 8 / R;
+    static_assert(R == 2 || R == 4 || R == 8, "a power of two");
+    C x[8];
+    zd_read<C, N, W, NS, R>(x, buf, tw, ev, w);
+    if constexpr (NS * R == N) {
+        // result j + r N / R of butterfly t is point m = t + r J
+#pragma unroll
+        for (int t = 0; t < J; t++) {
+#pragma unroll
+            for (int r = 0; r < R; r++) out[t + r * J] = x[t * R + r];
+        }
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < J; t++) {
+            const int j = ev + t * (N / 8), k = j % NS, d = (j / NS) * NS * R + k;
+#pragma unroll
+            for (int r = 0; r < R; r++) buf[(d + r * NS) * W + w] = x[t * R + r];
+        }
+        __syncthreads();
+        zd_stages<C, N, W, NS * R>(out, buf, tw, ev, w);
+    }
+}
+template <typename C, int N, int W, typename Then>
+__device__ __forceinline__ void zd_transform(C (&in)[8], C (&out)[8], C *buf, const C *tw, int ev, int w,
+                                             const Then &then) {
+    Butterfly<C, 8>::run(in);
+#pragma unroll
+    for (int r = 0; r < 8; r++) buf[(ev * 8 + r) * W + w] = in[r];
+    then();  // in is free
+    __syncthreads();
+    zd_stages<C, N, W, 8>(out, buf, tw, ev, w);
+}
+// a if c, else b (by value: a choice between array elements would put the
+// arrays into memory)
+template <typename C> __device__ __forceinline__ C pick(bool c, C a, C b) { return mk2<C>(c ? a.x : b.x, c ? a.y : b.y); }
+
+template <int N, int KIND, typename C>
+__global__ __launch_bounds__(zd_threads<N>()) void k_zsolve_direct(ZArgsT<C> A) {
+    constexpr int W = zd_cols<N>(), T = N * W / 8, NT = zd_threads<N>();
+    constexpr int NIN = ZSolve<KIND>::NIN, NOUT = ZSolve<KIND>::NOUT;
+    static_assert(NIN % 2 == 0, "whole rounds of inputs");
+    __shared__ C s_buf[2][N * W];
+    __shared__ C s_x[N * W];  // the halves that the groups trade
+    __shared__ C tw[N];
+    if (A.bt.cyc) {
+        const int b = blockIdx.z;
+        if (!gev::box_on(A.bt, b)) return;
+        const gev::BoxCycle &bc = A.bt.cyc[b];
+        A.in = gev::box_ptr(A.in, A.bt.stride, b);
+        A.out = gev::box_ptr(A.out, A.bt.stride, b);
+        A.bift = gev::box_ptr(A.bift, A.bt.stride, b);
+        A.kstore = gev::box_ptr(A.kstore, A.bt.stride, b);
+        A.k0 = gev::box_ptr(A.k0, A.bt.stride, b);
+        A.c0 = bc.a2dtau;
+    }
+    // XCD-aware tile order, as in k_zsolve
+    const int ntx = gridDim.x;
+    const int64_t NTL = (int64_t)ntx * gridDim.y;
+    int64_t L = (int64_t)blockIdx.y * ntx + blockIdx.x;
+    if (NTL % 8 == 0) L = (L % 8) * (NTL / 8) + L / 8;
+    const int kx0 = (int)(L % ntx) * W, ky = (int)(L / ntx);
+    const int64_t es = (int64_t)A.P * N;  // z stride
+    const int g = (int)threadIdx.x / T, tl = (int)threadIdx.x % T;
+    const int w = tl % W, ev = tl / W, kx = kx0 + w;
+    const bool ok = kx < A.H;
+    // point m of this thread: column base + m es N / 8 (the same for the whole
+    // workgroup) plus this thread's 32-bit byte offset
+    const int64_t base = (int64_t)ky * A.P + kx0;
+    const uint32_t off = (uint32_t)(((int64_t)ev * es + w) * (int64_t)sizeof(C));
+    auto point = [&](auto *p, int c, int m) __attribute__((always_inline)) {
+        using E = decltype(p);
+        char *const q = (char *)(p + (c * A.nkv + base + m * es * (N / 8)));
+        return (E)(q + off);
+    };
+    C *const buf = s_buf[g];
+    for (int t = threadIdx.x; t < N; t += NT) tw[t] = A.tw[t];
+
+    auto load = [&](int c, C (&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            v[m] = mk2<C>(0, 0);
+            if (ok) v[m] = *point(A.in, c, m);
+        }
+    };
+
+    // inputs: round r transforms components 2 r (group 0) and 2 r + 1
+    C S[NIN][4], v[8], X[8];
+    load(g, v);
+#pragma unroll
+    for (int r = 0; r < NIN / 2; r++) {
+        zd_transform<C, N, W>(v, X, buf, tw, ev, w, [&]() __attribute__((always_inline)) {
+            if (r + 1 < NIN / 2) load(2 * (r + 1) + g, v);
+        });
+        // group g keeps points 4 g .. 4 g + 3 of its component
+#pragma unroll
+        for (int i = 0; i < 4; i++) s_x[(g * 4 + i) * T + tl] = pick(g, X[i], X[4 + i]);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const C other = s_x[((1 - g) * 4 + i) * T + tl], own = pick(g, X[4 + i], X[i]);
+            S[2 * r][i] = pick(g, other, own);
+            S[2 * r + 1][i] = pick(g, own, other);
+        }
+    }
+
+    C O[NOUT][4];
+    const KRow row = k_row(A, kx, ky, ok);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int kz = ev + (4 * g + i) * (N / 8);
+        C Si[NIN], Oi[NOUT];
+#pragma unroll
+        for (int c = 0; c < NIN; c++) Si[c] = S[c][i];
+        solve_point<N, KIND, false>(A, row, kx, ky, kz, ok, base + w + (int64_t)kz * es, Si, (const C *)nullptr, Oi);
+#pragma unroll
+        for (int o = 0; o < NOUT; o++) O[o][i] = Oi[o];
+        __builtin_amdgcn_sched_barrier(0);  // one point at a time (registers)
+    }
+
+    // outputs: round r transforms back components 2 r and 2 r + 1 (those there are)
+#pragma unroll
+    for (int r = 0; r < (NOUT + 1) / 2; r++) {
+        const int oa = 2 * r, ob = 2 * r + 1 < NOUT ? 2 * r + 1 : 2 * r;  // group 0's and group 1's
+        if (r == 0) __syncthreads();  // the inputs' trade has been read
+#pragma unroll
+        for (int i = 0; i < 4; i++) s_x[(g * 4 + i) * T + tl] = pick(g, O[oa][i], O[ob][i]);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const C other = s_x[((1 - g) * 4 + i) * T + tl], own = pick(g, O[ob][i], O[oa][i]);
+            v[i] = cconj(pick(g, other, own));
+            v[4 + i] = cconj(pick(g, own, other));
+        }
+        zd_transform<C, N, W>(v, X, buf, tw, ev, w, []() {});
+        if (ok && 2 * r + g < NOUT) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) *point(A.out + (int64_t)g * A.nkv, 2 * r, m) = cconj(X[m]);
         }
     }
 }
@@ -518,11 +711,17 @@ template <int NC> int launch_x_nc(gev_ctx *c, XArgs A) {
 // ---------------------------------------------------------------- last pass
 
 template <int N, int KIND, typename C> int launch_n(gev_ctx *c, const ZArgsT<C> &A) {
-    constexpr int W = zs_cols<N, KIND, C>();
     const int H = N / 2 + 1;
     const unsigned nbox = A.bt.cyc ? (unsigned)c->nbox : 1u;
-    hipLaunchKernelGGL((k_zsolve<N, KIND, C>), dim3((H + W - 1) / W, N, nbox), dim3(zs_threads<N, KIND, C>()), 0,
-                       c->stream, A);
+    if constexpr (zd_direct<N, KIND, C>()) {
+        constexpr int W = zd_cols<N>();
+        hipLaunchKernelGGL((k_zsolve_direct<N, KIND, C>), dim3((H + W - 1) / W, N, nbox), dim3(zd_threads<N>()), 0,
+                           c->stream, A);
+    } else {
+        constexpr int W = zs_cols<N, KIND, C>();
+        hipLaunchKernelGGL((k_zsolve<N, KIND, C>), dim3((H + W - 1) / W, N, nbox), dim3(zs_threads<N, KIND, C>()), 0,
+                           c->stream, A);
+    }
     return gev::check_hip(c, hipGetLastError(), "fused z solve launch");
 }
 
