@@ -331,6 +331,32 @@ __global__ __launch_bounds__(TPB) void k_sort_cells(const uint32_t *__restrict__
     if (threadIdx.x == 0) flag[blockIdx.x] = big ? 1 : 0;
 }
 
+// The rank of entry i among the entries [b, f) by ID, ties by position.  The
+// loop over the keys is what the rank costs: IDs below 2^32 - 1 (those of any
+// lattice the grid sizes allow) are compared as 32-bit keys, one comparison
+// per key with the tie in its bound, and several keys in flight; larger and
+// negative IDs in 64 bits.  us per filing of a z = 0 state, 64-bit keys -> 32:
+// segments 512^3 1636 -> 1422, 384^3 798 -> 662, 256^3 301 -> 236, 128^3 71 ->
+// 44, 32^3 28 -> 16.  (Two rounds of registers instead of the LDS copies, four
+// 64-bit keys in flight: 256^3 346.)
+__device__ __forceinline__ bool wide_id(int64_t k) { return (uint64_t)k >= 0xffffffffull; }
+__device__ __forceinline__ uint32_t sort_rank(const int64_t *key, const uint32_t *k32, uint32_t b, uint32_t f,
+                                              uint32_t i, bool wide) {
+    uint32_t r = 0;
+    if (!wide) {
+        const uint32_t k = k32[i];
+#pragma unroll 4
+        for (uint32_t j = b; j < f; j++) r += k32[j] < k + (j < i ? 1u : 0u) ? 1u : 0u;
+    } else {
+        const int64_t k = key[i];
+        for (uint32_t j = b; j < f; j++) {
+            const int64_t kj = key[j];
+            r += (kj < k || (kj == k && j < i)) ? 1u : 0u;
+        }
+    }
+    return r;
+}
+
 // Workgroup b takes the flagged ones among segments b + k * gridDim.x,
 // k < SORT_SEG_BATCH (its first wave reads their flags at once): the larger
 // cells' entries are ranked in LDS, or, in a segment of more than SORT_SEG
@@ -354,7 +380,7 @@ __global__ __launch_bounds__(TPB) void k_sort_segments(const uint32_t *__restric
     nbig = gev::box_ptr(nbig, bt.stride, blockIdx.y);
     __shared__ int64_t s_key[SORT_SEG];
     __shared__ uint32_t s_val[SORT_SEG];
-    __shared__ uint32_t s_out[SORT_SEG];
+    __shared__ uint32_t s_k32[SORT_SEG];
     __shared__ uint32_t s_cs[TPB + 1];  // cell starts relative to the segment
     __shared__ uint8_t s_cell[SORT_SEG];  // each entry's cell in the segment
     __shared__ unsigned long long s_mask;
@@ -412,32 +438,27 @@ __global__ __launch_bounds__(TPB) void k_sort_segments(const uint32_t *__restric
             }
             return lo;
         };
+        // the segment's largest IDs decide how its IDs are compared (sort_rank)
+        bool wide = false;
         for (uint32_t i = threadIdx.x; i < total; i += TPB) {
             const int c = cell_of(i);
             s_cell[i] = (uint8_t)c;
             if (s_cs[c + 1] - s_cs[c] > SORT_TINY) {
                 const uint32_t v = perm[s0 + i];
+                const int64_t k = id[v];
                 s_val[i] = v;
-                s_key[i] = id[v];
+                s_key[i] = k;
+                s_k32[i] = (uint32_t)k;
+                wide |= wide_id(k);
             }
         }
-        __syncthreads();
+        wide = __syncthreads_or(wide);
         for (uint32_t i = threadIdx.x; i < total; i += TPB) {
             const int c = s_cell[i];
             const uint32_t b = s_cs[c] - sb, f = s_cs[c + 1] - sb;
             if (f - b <= SORT_TINY) continue;
-            const int64_t k = s_key[i];
-            uint32_t r = 0;
-            for (uint32_t j = b; j < f; j++) {
-                const int64_t kj = s_key[j];
-                r += (kj < k || (kj == k && j < i)) ? 1u : 0u;
-            }
-            s_out[b + r] = s_val[i];
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < total; i += TPB) {
-            const int c = s_cell[i];
-            if (s_cs[c + 1] - s_cs[c] > SORT_TINY) perm[s0 + i] = s_out[i];
+            const uint32_t r = sort_rank(s_key, s_k32, b, f, i, wide);
+            perm[s0 + b + r] = s_val[i];  // (the segment's entries have been read)
         }
         __syncthreads();  // the next segment rewrites s_cs and the copies
     }
@@ -458,6 +479,7 @@ __global__ __launch_bounds__(TPB) void k_sort_big(const uint32_t *__restrict__ s
     big = gev::box_ptr(big, bt.stride, blockIdx.y);
     nbig = gev::box_ptr(nbig, bt.stride, blockIdx.y);
     __shared__ int64_t s_key[SORT_LDS];
+    __shared__ uint32_t s_k32[SORT_LDS];
     __shared__ uint32_t s_val[SORT_LDS];
     const uint32_t nb = *nbig;
     for (uint32_t e = blockIdx.x; e < nb; e += gridDim.x) {
@@ -468,21 +490,18 @@ __global__ __launch_bounds__(TPB) void k_sort_big(const uint32_t *__restrict__ s
             __syncthreads();
             continue;
         }
+        bool wide = false;
         for (uint32_t i = threadIdx.x; i < m; i += TPB) {
             const uint32_t v = perm[b0 + i];
+            const int64_t k = id[v];
             s_val[i] = v;
-            s_key[i] = id[v];
+            s_key[i] = k;
+            s_k32[i] = (uint32_t)k;
+            wide |= wide_id(k);
         }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < m; i += TPB) {
-            const int64_t k = s_key[i];
-            uint32_t r = 0;
-            for (uint32_t j = 0; j < m; j++) {
-                const int64_t kj = s_key[j];
-                r += (kj < k || (kj == k && j < i)) ? 1u : 0u;
-            }
-            perm[b0 + r] = s_val[i];
-        }
+        wide = __syncthreads_or(wide);
+        for (uint32_t i = threadIdx.x; i < m; i += TPB)
+            perm[b0 + sort_rank(s_key, s_k32, 0u, m, i, wide)] = s_val[i];
         __syncthreads();  // the next cell overwrites the LDS copy
     }
 }

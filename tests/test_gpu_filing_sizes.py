@@ -32,3 +32,40 @@ def test_counts_and_order(gev, N, n):
             o = np.lexsort((ids, cell))
             assert np.array_equal(i, ids[o])
             assert np.array_equal(p, pos[o])
+
+
+def _wide_ids(rng, n, kind):
+    ids = rng.permutation(n).astype(np.int64)
+    if kind == "edge":  # the largest ID of the 32-bit comparison and the first beyond it
+        ids += 2 ** 32 - 2 - n // 2
+    elif kind == "mixed":  # beyond 32 bits with equal low words, negative, repeated
+        w = rng.random(n) < 0.3
+        ids[w] += rng.integers(-3, 4, w.sum()) << 32
+        ids[rng.integers(0, n, 50)] = ids[rng.integers(0, n, 50)]
+    else:  # every ID several times
+        ids //= 5
+    return ids
+
+
+@pytest.mark.parametrize("kind", ["edge", "mixed", "repeated"])
+def test_order_by_wide_and_repeated_ids(gev, kind):
+    N, n = 48, 60000
+    rng = np.random.default_rng(len(kind))
+    pos = rng.random((n, 3))
+    pos[:20000] = (rng.random((40, 3))[rng.integers(0, 40, 20000)] + 0.3 / N * rng.standard_normal((20000, 3))) % 1.0
+    pos[20000:21500] = 0.5 + 0.8 / N * rng.random((1500, 3))
+    pos[pos >= 1.0] = 0.0
+    ids = _wide_ids(rng, n, kind)
+    ci = np.floor(pos / (1.0 / N)).astype(np.int64)
+    cell = ci[:, 0] + N * (ci[:, 1] + N * ci[:, 2])
+    o = np.lexsort((ids, cell))
+    with gev.Box(N, n) as b:
+        b.upload_particles(pos, np.zeros((n, 3)), ids, 1.0)
+        b.moveParticles(gev.POS_NEWTON, 0.1, 0, [0.5, 0.25 * N])
+        p, _, i = b.download_particles()
+    assert np.array_equal(i, ids[o])
+    assert np.array_equal(np.sort(p, axis=0), np.sort(pos, axis=0))
+    # particles of one cell and ID may come in any order, others not
+    new = np.append(True, (np.diff(ids[o]) != 0) | (np.diff(cell[o]) != 0))
+    u = new & np.append(new[1:], True)
+    assert np.array_equal(p[u], pos[o][u])
