@@ -74,8 +74,10 @@ template <int N, int KIND, typename C> constexpr int zs_cols() {
 }
 // The tensor solve prefetches the carried B into registers during the last
 // input transform where the registers allow it; at N = 384 and above 512 the
-// prefetch would spill (compiler resource report), so B is read at the solve.
-// (FP32 form at 512^3: 3.04 against 3.21 ms with B read at the solve.)
+// prefetch would spill, and at N = 192 it would leave one wave per SIMD
+// (compiler resource report), so B is read at the solve.  (us per launch at
+// 192^3, prefetched -> read: FP64 393 -> 287, FP32 253 -> 184; FP32 form at
+// 512^3, where it fits: 3.04 against 3.21 ms with B read at the solve.)
 #ifndef GEV_ZS_AHEAD
 #define GEV_ZS_AHEAD 1
 #endif
@@ -84,7 +86,7 @@ constexpr int ZS_AHEAD = GEV_ZS_AHEAD;
 #define GEV_ZS_PREFETCH_F32 1
 #endif
 template <int N, typename C = double2> constexpr bool zs_prefetch_b() {
-    return ZS_AHEAD == 1 && N <= 512 && N != 384 && (GEV_ZS_PREFETCH_F32 || !is_f32<C>());
+    return ZS_AHEAD == 1 && N <= 512 && N != 192 && N != 384 && (GEV_ZS_PREFETCH_F32 || !is_f32<C>());
 }
 template <int N, int KIND, typename C> constexpr int zs_pts() {
     if (KIND != ZS_TENSOR && KIND != ZS_TENSOR_SCALAR) return 4;
@@ -116,86 +118,6 @@ template <typename C> struct ZArgsT {
     gev::Batch bt;       // over the boxes of a batch: box blockIdx.z, coefficients from its BoxCycle
 };
 using ZArgs = ZArgsT<double2>;
-
-// the k tables of a column
-struct KRow {
-    double gx, gy;
-    double2 kxs, kys;
-};
-template <typename C> __device__ __forceinline__ KRow k_row(const ZArgsT<C> &A, int kx, int ky, bool ok) {
-    return KRow{A.g[ok ? kx : 0], A.g[ky], A.ks[ok ? kx : 0], A.ks[ky]};
-}
-
-// The solve of one k point (kx, ky, kz) from its transformed inputs S, in
-// FP64 (the FP32 form's tensor solves: FP64 coefficients and denominators,
-// float field combinations); the outputs O are kept in the storage type (k = 0
-// of output 0 also in FP64).  at: the point's index in a k field.  HAVE_B: Bo
-// holds the carried B of the point, otherwise it is read here.
-template <int N, int KIND, bool HAVE_B, typename C>
-__device__ __forceinline__ void solve_point(const ZArgsT<C> &A, const KRow &row, int kx, int ky, int kz, bool live,
-                                            int64_t at, const C *S, const C *Bo, C *O) {
-    const double gx = row.gx, gy = row.gy, gz = A.g[live ? kz : 0];
-    const double2 kxs = row.kxs, kys = row.kys, kzs = A.ks[live ? kz : 0];
-    const bool zero = kx == 0 && ky == 0 && kz == 0;
-    auto carried = [&](int c) { return HAVE_B ? Bo[c] : A.bift[c * A.nkv + at]; };
-    double2 o0;
-    if constexpr (KIND == ZS_POISSON) {
-        o0 = poisson_point(d2(S[0]), zero, zero ? 0. : gx + gy + gz, A.c0, A.c1);
-    } else if constexpr ((KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) && is_f32<C>()) {
-        const float2 chi = zero ? make_float2(0.f, 0.f) : project_scalar_f32(S, gx, gy, gz, kxs, kys, kzs, N);
-        o0 = make_double2(chi.x, chi.y);
-        if constexpr (KIND == ZS_TENSOR) {
-            float2 B[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-            if (live) {
-                if (!zero) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) B[c] = carried(c);
-                    evolve_vector_f32(S, B, gx, gy, gz, kxs, kys, kzs, A.c0);
-                }
-#pragma unroll
-                for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = B[c];
-            }
-#pragma unroll
-            for (int c = 0; c < 3; c++) O[1 + c] = B[c];
-        }
-    } else if constexpr (KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) {
-        double2 Sp[6];
-#pragma unroll
-        for (int c = 0; c < 6; c++) Sp[c] = d2(S[c]);
-        o0 = zero ? c2(0., 0.) : project_scalar(Sp, gx, gy, gz, kxs, kys, kzs, N);
-        if constexpr (KIND == ZS_TENSOR) {
-            double2 B[3] = {c2(0., 0.), c2(0., 0.), c2(0., 0.)};
-            if (live) {
-                if (!zero) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++) B[c] = d2(carried(c));
-                    evolve_vector(Sp, B, gx, gy, gz, kxs, kys, kzs, A.c0);
-                }
-#pragma unroll
-                for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = from_d2<C>(B[c]);
-            }
-#pragma unroll
-            for (int c = 0; c < 3; c++) O[1 + c] = from_d2<C>(B[c]);
-        }
-    } else {
-        double2 Sv[3] = {d2(S[0]), d2(S[1]), d2(S[2])};
-        if (zero) {
-            Sv[0] = Sv[1] = Sv[2] = c2(0., 0.);
-        } else {
-            project_vector_point(Sv, kxs, kys, kzs, gx + gy + gz, A.c0, A.c1);
-        }
-        if (live && A.bift) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = from_d2<C>(Sv[c]);
-        }
-        o0 = Sv[0];
-#pragma unroll
-        for (int c = 1; c < 3; c++) O[c] = from_d2<C>(Sv[c]);
-    }
-    O[0] = from_d2<C>(o0);
-    if (live && A.kstore) A.kstore[at] = O[0];
-    if (zero && A.k0) A.k0[0] = o0;
-}
 
 template <int N, int KIND, typename C>
 __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C> A) {
@@ -294,25 +216,100 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
         }
     }
 
-    // the solve, per k point (kx, ky, kz = element index)
+    // the solve, per k point (kx, ky, kz = element index), in FP64; the
+    // outputs are kept in the storage type (k = 0 of output 0 also in FP64)
     C O[NOUT][PTS];
-    const KRow row = k_row(A, kx, ky, ok);
+    const double gx = A.g[ok ? kx : 0];
+    const double2 kxs = A.ks[ok ? kx : 0];
+    const double gy = A.g[ky];
+    const double2 kys = A.ks[ky];
 #pragma unroll
     for (int j = 0; j < PTS; j++) {
         const int idx = threadIdx.x + j * NT;
         const int kz = idx / W;
         const bool live = ok && (EXACT || idx < N * W);
-        C Sj[NIN], Oj[NOUT], Bj[3];
+        const double gz = A.g[live ? kz : 0];
+        const double2 kzs = A.ks[live ? kz : 0];
+        const bool zero = kx == 0 && ky == 0 && kz == 0;
+        const int64_t at = base + (int64_t)kz * es + w;
+        double2 o0;
+        if constexpr (KIND == ZS_POISSON) {
+            o0 = poisson_point(d2(S[0][j]), zero, zero ? 0. : gx + gy + gz, A.c0, A.c1);
+        } else if constexpr ((KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) && is_f32<C>()) {
+            // FP32 form: FP64 coefficients and denominators, float field combinations
+            float2 Sf[6];
 #pragma unroll
-        for (int c = 0; c < NIN; c++) Sj[c] = S[c][j];
-        if constexpr (KIND == ZS_TENSOR && zs_prefetch_b<N, C>()) {
+            for (int c = 0; c < 6; c++) Sf[c] = S[c][j];
+            const float2 chi = zero ? make_float2(0.f, 0.f) : project_scalar_f32(Sf, gx, gy, gz, kxs, kys, kzs, N);
+            o0 = make_double2(chi.x, chi.y);
+            if constexpr (KIND == ZS_TENSOR) {
+                float2 B[3] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+                if (live) {
+                    if (!zero) {
+                        if constexpr (zs_prefetch_b<N, C>()) {
+                            B[0] = Bold[0][j];
+                            B[1] = Bold[KIND == ZS_TENSOR ? 1 : 0][j];
+                            B[2] = Bold[KIND == ZS_TENSOR ? 2 : 0][j];
+                        } else {
+                            B[0] = A.bift[at];
+                            B[1] = A.bift[A.nkv + at];
+                            B[2] = A.bift[2 * A.nkv + at];
+                        }
+                        evolve_vector_f32(Sf, B, gx, gy, gz, kxs, kys, kzs, A.c0);
+                    }
+                    A.bift[at] = B[0];
+                    A.bift[A.nkv + at] = B[1];
+                    A.bift[2 * A.nkv + at] = B[2];
+                }
 #pragma unroll
-            for (int c = 0; c < 3; c++) Bj[c] = Bold[c][j];
+                for (int c = 0; c < 3; c++) O[1 + c][j] = B[c];
+            }
+        } else if constexpr (KIND == ZS_TENSOR || KIND == ZS_TENSOR_SCALAR) {
+            double2 Sp[6];
+#pragma unroll
+            for (int c = 0; c < 6; c++) Sp[c] = d2(S[c][j]);
+            o0 = zero ? c2(0., 0.) : project_scalar(Sp, gx, gy, gz, kxs, kys, kzs, N);
+            if constexpr (KIND == ZS_TENSOR) {
+                double2 B[3] = {c2(0., 0.), c2(0., 0.), c2(0., 0.)};
+                if (live) {
+                    if (!zero) {
+                        if constexpr (zs_prefetch_b<N, C>()) {
+                            B[0] = d2(Bold[0][j]);
+                            B[1] = d2(Bold[KIND == ZS_TENSOR ? 1 : 0][j]);
+                            B[2] = d2(Bold[KIND == ZS_TENSOR ? 2 : 0][j]);
+                        } else {
+                            B[0] = d2(A.bift[at]);
+                            B[1] = d2(A.bift[A.nkv + at]);
+                            B[2] = d2(A.bift[2 * A.nkv + at]);
+                        }
+                        evolve_vector(Sp, B, gx, gy, gz, kxs, kys, kzs, A.c0);
+                    }
+                    A.bift[at] = from_d2<C>(B[0]);
+                    A.bift[A.nkv + at] = from_d2<C>(B[1]);
+                    A.bift[2 * A.nkv + at] = from_d2<C>(B[2]);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) O[1 + c][j] = from_d2<C>(B[c]);
+            }
+        } else {
+            double2 Sv[3] = {d2(S[0][j]), d2(S[1][j]), d2(S[2][j])};
+            if (zero) {
+                Sv[0] = Sv[1] = Sv[2] = c2(0., 0.);
+            } else {
+                project_vector_point(Sv, kxs, kys, kzs, gx + gy + gz, A.c0, A.c1);
+            }
+            if (live && A.bift) {
+                A.bift[at] = from_d2<C>(Sv[0]);
+                A.bift[A.nkv + at] = from_d2<C>(Sv[1]);
+                A.bift[2 * A.nkv + at] = from_d2<C>(Sv[2]);
+            }
+            o0 = Sv[0];
+#pragma unroll
+            for (int c = 1; c < 3; c++) O[c][j] = from_d2<C>(Sv[c]);
         }
-        solve_point<N, KIND, (KIND == ZS_TENSOR && zs_prefetch_b<N, C>())>(A, row, kx, ky, kz, live,
-                                                                           base + (int64_t)kz * es + w, Sj, Bj, Oj);
-#pragma unroll
-        for (int o = 0; o < NOUT; o++) O[o][j] = Oj[o];
+        O[0][j] = from_d2<C>(o0);
+        if (live && A.kstore) A.kstore[at] = O[0][j];
+        if (zero && A.k0) A.k0[0] = o0;
     }
 
     // inverse z transform of every output (conjugate, forward stages, conjugate)
@@ -336,7 +333,8 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
 
 // ---------------------------------------------------------------- direct form
 //
-// The FP64 tensor solve with the carried B, for powers of two from 64.  A
+// The FP64 tensor solve with the carried B, for powers of two from 64 to 512 (at
+// 1024 it spills).  A
 // transform's first stage reads, and its last stage leaves, 8 points of a
 // column per thread: kz = ev + m N / 8 (m < 8, ev = its butterfly).  The loads,
 // the solve, the inverse transform's first stage and the stores work on these
@@ -348,18 +346,16 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
 // k_zsolve, and two components' loads in flight.
 // Bound by the latency of its loads and barriers at 8 waves per CU (the
 // registers; 3 TB/s at 512^3).  us per launch, k_zsolve -> this: 512^3 4756 ->
-// 4640, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.7 -> 17.4, 32^3 12.1
+// 4685, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.9 -> 16.5, 32^3 12.1
 // both.  FP32 stays on k_zsolve: its float points leave a thread room for 8
 // points of all components only with spills (512^3 3012 -> 3432, 256^3 344 ->
 // 572); so do the FP64 solves with fewer fields (Poisson 512^3 620 -> 636, chi
 // alone 256^3 294 -> 305).
 template <int N, int KIND, typename C> constexpr bool zd_direct() {
-    return !is_f32<C>() && KIND == ZS_TENSOR && N >= 64 && (N & (N - 1)) == 0;
+    return !is_f32<C>() && KIND == ZS_TENSOR && N >= 64 && N <= 512 && (N & (N - 1)) == 0;
 }
-// columns per workgroup: 64-byte rows where the two buffers and the traded
-// halves fit LDS
-template <int N> constexpr int zd_cols() { return N >= 1024 ? 2 : 4; }
-template <int N> constexpr int zd_threads() { return 2 * N * zd_cols<N>() / 8; }
+constexpr int ZD_COLS = 4;  // columns per workgroup: 64-byte rows
+template <int N> constexpr int zd_threads() { return 2 * N * ZD_COLS / 8; }
 
 // The transform of 8 points per thread (column w, points ev + m N / 8) of
 // N x W points in LDS; then() runs once the inputs are in LDS.  The caller
@@ -417,11 +413,12 @@ __device__ __forceinline__ void zd_transform(C (&in)[8], C (&out)[8], C *buf, co
 // arrays into memory)
 template <typename C> __device__ __forceinline__ C pick(bool c, C a, C b) { return mk2<C>(c ? a.x : b.x, c ? a.y : b.y); }
 
-template <int N, int KIND, typename C>
-__global__ __launch_bounds__(zd_threads<N>()) void k_zsolve_direct(ZArgsT<C> A) {
-    constexpr int W = zd_cols<N>(), T = N * W / 8, NT = zd_threads<N>();
-    constexpr int NIN = ZSolve<KIND>::NIN, NOUT = ZSolve<KIND>::NOUT;
-    static_assert(NIN % 2 == 0, "whole rounds of inputs");
+template <int N>
+__global__ __launch_bounds__(zd_threads<N>()) void k_zsolve_direct(ZArgs A) {
+    using C = double2;
+    constexpr int W = ZD_COLS, T = N * W / 8, NT = zd_threads<N>();
+    constexpr int NIN = ZSolve<ZS_TENSOR>::NIN, NOUT = ZSolve<ZS_TENSOR>::NOUT;
+    static_assert(NIN == 6 && NOUT == 4, "three rounds in, two out");
     __shared__ C s_buf[2][N * W];
     __shared__ C s_x[N * W];  // the halves that the groups trade
     __shared__ C tw[N];
@@ -486,24 +483,41 @@ __global__ __launch_bounds__(zd_threads<N>()) void k_zsolve_direct(ZArgsT<C> A) 
         }
     }
 
+    // the solve, point by point as in k_zsolve
     C O[NOUT][4];
-    const KRow row = k_row(A, kx, ky, ok);
+    const double gx = A.g[ok ? kx : 0], gy = A.g[ky];
+    const double2 kxs = A.ks[ok ? kx : 0], kys = A.ks[ky];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int kz = ev + (4 * g + i) * (N / 8);
-        C Si[NIN], Oi[NOUT];
+        const double gz = A.g[ok ? kz : 0];
+        const double2 kzs = A.ks[ok ? kz : 0];
+        const bool zero = kx == 0 && ky == 0 && kz == 0;
+        const int64_t at = base + w + (int64_t)kz * es;
+        double2 Sp[6], B[3] = {c2(0., 0.), c2(0., 0.), c2(0., 0.)};
 #pragma unroll
-        for (int c = 0; c < NIN; c++) Si[c] = S[c][i];
-        solve_point<N, KIND, false>(A, row, kx, ky, kz, ok, base + w + (int64_t)kz * es, Si, (const C *)nullptr, Oi);
+        for (int c = 0; c < 6; c++) Sp[c] = S[c][i];
+        O[0][i] = zero ? c2(0., 0.) : project_scalar(Sp, gx, gy, gz, kxs, kys, kzs, N);
+        if (ok) {
+            if (!zero) {
 #pragma unroll
-        for (int o = 0; o < NOUT; o++) O[o][i] = Oi[o];
+                for (int c = 0; c < 3; c++) B[c] = A.bift[c * A.nkv + at];
+                evolve_vector(Sp, B, gx, gy, gz, kxs, kys, kzs, A.c0);
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) A.bift[c * A.nkv + at] = B[c];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) O[1 + c][i] = B[c];
+        if (ok && A.kstore) A.kstore[at] = O[0][i];
+        if (zero && A.k0) A.k0[0] = O[0][i];
         __builtin_amdgcn_sched_barrier(0);  // one point at a time (registers)
     }
 
-    // outputs: round r transforms back components 2 r and 2 r + 1 (those there are)
+    // outputs: round r transforms back components 2 r and 2 r + 1
 #pragma unroll
-    for (int r = 0; r < (NOUT + 1) / 2; r++) {
-        const int oa = 2 * r, ob = 2 * r + 1 < NOUT ? 2 * r + 1 : 2 * r;  // group 0's and group 1's
+    for (int r = 0; r < NOUT / 2; r++) {
+        const int oa = 2 * r, ob = 2 * r + 1;  // group 0's and group 1's
         if (r == 0) __syncthreads();  // the inputs' trade has been read
 #pragma unroll
         for (int i = 0; i < 4; i++) s_x[(g * 4 + i) * T + tl] = pick(g, O[oa][i], O[ob][i]);
@@ -515,7 +529,7 @@ __global__ __launch_bounds__(zd_threads<N>()) void k_zsolve_direct(ZArgsT<C> A) 
             v[4 + i] = cconj(pick(g, own, other));
         }
         zd_transform<C, N, W>(v, X, buf, tw, ev, w, []() {});
-        if (ok && 2 * r + g < NOUT) {
+        if (ok) {
 #pragma unroll
             for (int m = 0; m < 8; m++) *point(A.out + (int64_t)g * A.nkv, 2 * r, m) = cconj(X[m]);
         }
@@ -714,8 +728,8 @@ template <int N, int KIND, typename C> int launch_n(gev_ctx *c, const ZArgsT<C> 
     const int H = N / 2 + 1;
     const unsigned nbox = A.bt.cyc ? (unsigned)c->nbox : 1u;
     if constexpr (zd_direct<N, KIND, C>()) {
-        constexpr int W = zd_cols<N>();
-        hipLaunchKernelGGL((k_zsolve_direct<N, KIND, C>), dim3((H + W - 1) / W, N, nbox), dim3(zd_threads<N>()), 0,
+        constexpr int W = ZD_COLS;
+        hipLaunchKernelGGL(k_zsolve_direct<N>, dim3((H + W - 1) / W, N, nbox), dim3(zd_threads<N>()), 0,
                            c->stream, A);
     } else {
         constexpr int W = zs_cols<N, KIND, C>();
