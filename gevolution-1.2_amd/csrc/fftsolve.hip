@@ -333,24 +333,26 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
 
 // ---------------------------------------------------------------- direct form
 //
-// The FP64 tensor solve with the carried B, for powers of two from 64 to 512 (at
-// 1024 it spills).  A
-// transform's first stage reads, and its last stage leaves, 8 points of a
-// column per thread: kz = ev + m N / 8 (m < 8, ev = its butterfly).  The loads,
-// the solve, the inverse transform's first stage and the stores work on these
-// registers, and LDS carries only the exchanges between stages (2 round trips
-// per transform at N = 512 where k_zsolve makes 4).  6 components x 8 points
-// do not fit the registers of a thread: the workgroup is two groups of threads
-// that transform two components at once and trade halves through LDS, so that
-// each thread solves 4 points of all components; half as many barriers as
-// k_zsolve, and two components' loads in flight.
+// The FP64 tensor solve with the carried B, for powers of two from 64 to 512
+// (at 1024 it spills).  A transform's first stage reads, and its last stage
+// leaves, 8 points of a column per thread: kz = ev + m N / 8 (m < 8, ev = its
+// butterfly).  The loads, the solve, the inverse transform's first stage and
+// the stores work on these registers, and LDS carries only the exchanges
+// between stages (2 round trips per transform at N = 512 where k_zsolve makes
+// 4).  6 components x 8 points do not fit the registers of a thread: the
+// workgroup is two groups of threads that transform two components at once and
+// trade halves through LDS, so that each thread solves 4 points of all
+// components; half as many barriers as k_zsolve, and two components' loads in
+// flight.
 // Bound by the latency of its loads and barriers at 8 waves per CU (the
-// registers; 3 TB/s at 512^3).  us per launch, k_zsolve -> this: 512^3 4756 ->
-// 4685, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.9 -> 16.5, 32^3 12.1
+// registers; 3.7 TB/s at 512^3).  us per launch, k_zsolve -> this: 512^3 4756
+// -> 4685, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.9 -> 16.5, 32^3 12.1
 // both.  FP32 stays on k_zsolve: its float points leave a thread room for 8
 // points of all components only with spills (512^3 3012 -> 3432, 256^3 344 ->
-// 572); so do the FP64 solves with fewer fields (Poisson 512^3 620 -> 636, chi
-// alone 256^3 294 -> 305).
+// 572); so do the FP64 solves with fewer fields, which gain nothing (Poisson
+// 512^3 620 -> 636, chi alone 256^3 294 -> 305).  The solve of a point stands in
+// both kernels: as a shared function it cost k_zsolve registers (FP32 256^3
+// 337 -> 466).
 template <int N, int KIND, typename C> constexpr bool zd_direct() {
     return !is_f32<C>() && KIND == ZS_TENSOR && N >= 64 && N <= 512 && (N & (N - 1)) == 0;
 }
