@@ -260,7 +260,7 @@ template <int N> constexpr int x_lines() {
 }
 
 // columns per workgroup of the strided passes: GEV_COL_BYTES-byte rows
-// (default 128), at most 64 KiB
+// (default 128), at most 64 KiB (96 at N = 768 in FP64, see col_tpb)
 #ifndef GEV_COL_BYTES
 #define GEV_COL_BYTES 128
 #endif
@@ -271,20 +271,25 @@ template <int N> constexpr int x_lines() {
 // batch may pick 64 or 256 instead
 template <typename T, int N, int RB = 0> constexpr int col_tile() {
     int w = (RB ? RB : (sizeof(T) == 4 ? GEV_COL_BYTES_F32 : GEV_COL_BYTES)) / (int)(2 * sizeof(T));
-    while (w > 1 && w * N * (int)(2 * sizeof(T)) > 65536) w /= 2;
+    while (w > 1 && w * N * (int)(2 * sizeof(T)) > (N == 768 && sizeof(T) == 8 ? 98304 : 65536)) w /= 2;
     return w;
 }
 // Threads per workgroup of the strided passes: one first-stage butterfly
 // each (a small tile takes a small workgroup, so more tiles share a CU), at
-// most GEV_COL_TPB / GEV_COL_TPB_F32 threads with several each.
+// most GEV_COL_TPB / GEV_COL_TPB_F32 threads with several each.  At N = 768
+// one each too, 768 threads: with two each the passes leave too few wavefronts
+// for their loads (us per pass, y / z, two each -> one: FP32 1024 / 1180 -> 785
+// / 890; FP64, where the tile grows to 128-byte rows with it, 1630 / 1850 ->
+// 1555 / 1700.  One each on 64-byte rows in FP64: 1835 / 2140), and at 384 in
+// FP32 (111 / 69 -> 102 / 67; in FP64 169 / 197 -> 200 / 219, left at two).
 #ifndef GEV_COL_TPB
 #define GEV_COL_TPB 256
 #endif
 #ifndef GEV_COL_TPB_F32
-#define GEV_COL_TPB_F32 512
+#define GEV_COL_TPB_F32 768
 #endif
 template <typename T, int N, int RB = 0> constexpr int col_tpb() {
-    constexpr int cap = sizeof(T) == 4 ? GEV_COL_TPB_F32 : GEV_COL_TPB;
+    constexpr int cap = sizeof(T) == 4 ? GEV_COL_TPB_F32 : N == 768 ? 768 : GEV_COL_TPB;
     constexpr int jobs = N / next_radix(N) * col_tile<T, N, RB>(), k = (jobs + cap - 1) / cap;
     return ((jobs + k - 1) / k + 63) / 64 * 64;
 }
