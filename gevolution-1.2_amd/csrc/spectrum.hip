@@ -59,29 +59,36 @@ template <typename C> __device__ __forceinline__ double cross(const PkArgsT<C> &
     return p;
 }
 
-// A workgroup takes four rows at a time.  Each of its wavefronts forms one
-// row's terms in LDS and lists where the runs begin; then a lane sums one run
-// in kx order, run i of the four rows in neighbouring lanes, so the long runs
-// near kx = 0 (up to about 35 modes; 3 beyond) share a wavefront; then
-// wavefront q folds quantity q of the four rows into the histogram, row after
-// row.  The sums and their order are those of one mode after another.  Bound
-// by the instructions of the terms (FP64 roots and divisions) and of the
-// serial sums: with k_spectrum_reduce 1.33 ms at 512^3, 0.12 at 192^3, 26 us
-// at 64^3 (one row at a time per workgroup, and a serial column of loads per
-// thread in k_spectrum_reduce: 1.84, 0.38 and 0.23 ms).  Passing the sums
-// from lane to lane by shuffles took 3.2 ms at 512^3.
+// A workgroup takes ROWS rows at a time.  Its wavefronts form the rows' terms
+// in LDS (one row each, or two to a row) and one per row lists where the runs
+// begin; then a lane sums one run in kx order, run i of the rows in
+// neighbouring lanes, so the long runs near kx = 0 (up to about 35 modes; 3
+// beyond) share a wavefront; then wavefront q folds quantity q of the rows
+// into the histogram, row after row.  The sums and their order are those of
+// one mode after another.  Bound by the instructions of the terms (FP64 roots
+// and divisions) and of the serial sums: with k_spectrum_reduce 1.33 ms at
+// 512^3, 0.12 at 192^3, 26 us at 64^3 (one row at a time per workgroup, and a
+// serial column of loads per thread in k_spectrum_reduce: 1.84, 0.38 and 0.23
+// ms).  Passing the sums from lane to lane by shuffles took 3.2 ms at 512^3.
 // Occupations are whole numbers, added with LDS atomics in any order.
-template <int MAXH, typename C>
+template <int MAXH, int ROWS, typename C>
 __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
     constexpr int WAVES = TPB / 64, J = (MAXH + 63) / 64;
+    constexpr int PER_ROW = WAVES / ROWS;  // wavefronts that form one row's terms
     static_assert(WAVES == NQ - 1, "a wavefront per summed quantity");
+    static_assert(PER_ROW * ROWS == WAVES, "the wavefronts share the rows evenly");
     extern __shared__ double hist[];  // (NQ - 1) * numbins sums, then numbins counts (uint32)
     __shared__ double s_tk[MAXH];                // typek2 of kx
-    __shared__ double s_q[3][WAVES][MAXH];       // weight * (k, P k^3 / s, (P k^3 / s)^2); a run's sum at its head
-    __shared__ double s_q1[WAVES][MAXH];         // a run's sum of weight * k^2 at its head
-    __shared__ int16_t s_bin[WAVES][MAXH];
-    __shared__ int16_t s_run[WAVES][MAXH + 1];   // where the runs begin (runs outside the bins too), and the end
-    __shared__ int s_n[WAVES];
+    __shared__ double s_q[3][ROWS][MAXH];        // weight * (k, P k^3 / s, (P k^3 / s)^2); a run's sums at its head
+    // A run's sum of weight * k^2 has a table of its own, at its head; on long
+    // rows, to save that LDS, it stands behind the sum of weight * k (a run of
+    // one mode has no room for it and no sum to keep)
+    constexpr bool OWN_Q1 = MAXH <= 257;
+    __shared__ double s_q1[OWN_Q1 ? ROWS : 1][OWN_Q1 ? MAXH : 1];
+    __shared__ int16_t s_bin[ROWS][MAXH];
+    __shared__ int16_t s_run[ROWS][MAXH + 1];   // where the runs begin (runs outside the bins too), and the end
+    __shared__ int s_n[ROWS];
+    __shared__ double s_ty[ROWS], s_tz[ROWS];    // typek2 of the rows' ky and kz
     uint32_t *const count = reinterpret_cast<uint32_t *>(hist + (NQ - 1) * A.numbins);
     const int N = A.N, H = N / 2, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int t = threadIdx.x; t < A.numbins * (NQ - 1); t += TPB) hist[t] = 0.;
@@ -90,15 +97,27 @@ __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
     const int64_t r0 = (int64_t)blockIdx.x * A.rows_per_block;
     const int64_t r1 = min(r0 + A.rows_per_block, (int64_t)N * N);
     auto weight_of = [&](int kx) { return (kx == 0 || (kx == N / 2 && N % 2 == 0)) ? 1 : 2; };
-    for (int64_t rg = r0; rg < r1; rg += WAVES) {
+    // the runs of row q from the bins of the 64 modes from kb on, n of them so
+    // far; last: the bin of the mode before these
+    auto list_runs = [&](int q, int kb, int bin, int &n, int &last) {
+        const int up = __shfl_up(bin, 1);
+        const bool head = kb + lane <= H && bin != (lane == 0 ? last : up);
+        const uint64_t heads = __ballot(head);
+        if (head) s_run[q][n + (int)__popcll(heads & ((1ull << lane) - 1ull))] = (int16_t)(kb + lane);
+        n += (int)__popcll(heads);
+        last = __shfl(bin, 63);
+    };
+    for (int64_t rg = r0; rg < r1; rg += ROWS) {
         __syncthreads();  // the tables are there, the previous rows are folded
-        const int64_t r = rg + wave;
-        int n = 0;  // runs of this row
+        const int q = wave % ROWS;
+        const int64_t r = rg + q;
+        int n = 0, last = -2;  // runs of this row
+        double tky = 0., tkz = 0.;
         if (r < r1) {
             const int ky = (int)(r % N), kz = (int)(r / N);
-            const double tky = A.typek2[ky], tkz = A.typek2[kz], sky = A.sinc[ky], skz = A.sinc[kz];
-            int open = -2;  // the bin of the mode before these 64
-            for (int kb = 0; kb <= H; kb += 64) {
+            const double sky = A.sinc[ky], skz = A.sinc[kz];
+            tky = A.typek2[ky], tkz = A.typek2[kz];
+            for (int kb = wave / ROWS * 64; kb <= H; kb += 64 * PER_ROW) {
                 const int kx = kb + lane;
                 int bin = -1;
                 if (kx <= H) {
@@ -117,38 +136,41 @@ __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
                             q3 = weight * p * p * k2 * k2 * k2 / s / s;
                         }
                     }
-                    s_bin[wave][kx] = (int16_t)bin;
-                    s_q[0][wave][kx] = q0;
-                    s_q[1][wave][kx] = q2;
-                    s_q[2][wave][kx] = q3;
+                    s_bin[q][kx] = (int16_t)bin;
+                    s_q[0][q][kx] = q0;
+                    s_q[1][q][kx] = q2;
+                    s_q[2][q][kx] = q3;
                 }
-                const int up = __shfl_up(bin, 1);
-                const bool head = kx <= H && bin != (lane == 0 ? open : up);
-                const uint64_t heads = __ballot(head);
-                if (head) s_run[wave][n + (int)__popcll(heads & ((1ull << lane) - 1ull))] = (int16_t)kx;
-                n += (int)__popcll(heads);
-                open = __shfl(bin, 63);
+                if (PER_ROW == 1) list_runs(q, kb, bin, n, last);
             }
-            if (lane == 0) s_run[wave][n] = (int16_t)(H + 1);
         }
-        if (lane == 0) s_n[wave] = n;
+        if (PER_ROW > 1) {
+            __syncthreads();  // the rows' bins are there
+            if (wave < ROWS && r < r1)
+                for (int kb = 0; kb <= H; kb += 64)
+                    list_runs(q, kb, kb + lane <= H ? (int)s_bin[q][kb + lane] : -1, n, last);
+        }
+        if (wave < ROWS && lane == 0) {
+            s_run[q][n] = (int16_t)(H + 1);
+            s_n[q] = n;
+            s_ty[q] = tky;
+            s_tz[q] = tkz;
+        }
         __syncthreads();
         int most = 0;
 #pragma unroll
-        for (int w = 0; w < WAVES; w++) most = max(most, s_n[w]);
-        for (int t = threadIdx.x; t < most * WAVES; t += TPB) {
-            const int w = t % WAVES, i = t / WAVES;
+        for (int w = 0; w < ROWS; w++) most = max(most, s_n[w]);
+        for (int t = threadIdx.x; t < most * ROWS; t += TPB) {
+            const int w = t % ROWS, i = t / ROWS;
             if (i >= s_n[w]) continue;
             const int b = s_run[w][i], e = s_run[w][i + 1], bin = s_bin[w][b];
             if (bin < 0) continue;
-            const int64_t row = rg + w;
-            const double tky = A.typek2[row % N], tkz = A.typek2[row / N];
             double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
             uint32_t m = 0;
 #pragma unroll 2
             for (int k = b; k < e; k++) {
                 const int weight = weight_of(k);
-                const double k2 = s_tk[k] + tky + tkz;
+                const double k2 = s_tk[k] + s_ty[w] + s_tz[w];
                 a0 += s_q[0][w][k];
                 a1 += weight * k2;
                 a2 += s_q[1][w][k];
@@ -157,15 +179,16 @@ __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
             }
             // (a run's terms are read by this lane alone)
             s_q[0][w][b] = a0;
-            s_q1[w][b] = a1;
+            if constexpr (OWN_Q1) s_q1[w][b] = a1;
+            else if (e - b > 1) s_q[0][w][b + 1] = a1;
             s_q[1][w][b] = a2;
             s_q[2][w][b] = a3;
             atomicAdd(count + bin, m);
         }
         __syncthreads();
-        const double(*const src)[MAXH] = wave == 0 ? s_q[0] : wave == 1 ? s_q1 : wave == 2 ? s_q[1] : s_q[2];
+        const double(*const src)[MAXH] = s_q[max(wave - 1, 0)];
         double *const h = hist + wave * A.numbins;
-        for (int w = 0; w < WAVES; w++) {
+        for (int w = 0; w < ROWS; w++) {
             // no two runs of a row share a bin: read, add and write them side by side
             const int m = s_n[w];
             int bin[J];
@@ -177,7 +200,10 @@ __global__ __launch_bounds__(TPB) void k_spectrum_rows(PkArgsT<C> A) {
                 if (lane + 64 * j < m) {
                     const int b = s_run[w][lane + 64 * j];
                     bin[j] = s_bin[w][b];
-                    v[j] = src[w][b];
+                    if (wave != 1) v[j] = src[w][b];
+                    else if constexpr (OWN_Q1) v[j] = s_q1[w][b];
+                    else if (s_run[w][lane + 64 * j + 1] - b > 1) v[j] = src[w][b + 1];
+                    else v[j] = weight_of(b) * (s_tk[b] + s_ty[w] + s_tz[w]);
                 }
             }
 #pragma unroll
@@ -275,12 +301,31 @@ int64_t spectrum_scratch_doubles(int N, int numbins) {
     return 2 * (int64_t)N + ((int64_t)nblk + 1) * numbins * NQ;
 }
 
-// the row kernel with LDS for the rows of its grid size (more workgroups per CU on smaller grids)
+// The row kernel with LDS for the rows of its grid size (more workgroups per
+// CU on smaller grids).  Four rows at a time, so that more of the long runs
+// share a wavefront, unless they and the bins leave a CU one workgroup (above
+// 700 bins on rows of up to 385 modes, above 550 on longer ones): then two.
+// ms with k_spectrum_reduce, two rows / four / four with room for 513 modes
+// and a table of its own for the k^2 sums on all long rows: 768^3 FP32 with 16
+// bins 6.1 / 4.7 / 5.4, with 384 3.4 / 4.1 / 7.3, with 1024 6.1 / - / 8.0;
+// 1024^3 with 64 bins 8.1 / 9.5 / 9.5, with 512 10.8 / 9.2 / 15.8, with 1024
+// 12.6 / - / 17.1.
+template <int MAXH, typename C> static void launch_rows_of(gev_ctx *c, const PkArgsT<C> &A, int nblk, size_t shm) {
+    constexpr size_t four = 4 * MAXH * (3 * 8 + 2 * 2) + MAXH * 8 + 256, half_lds = 160 * 1024 / 2;
+    if constexpr (MAXH > 257) {
+        if (four + shm > half_lds) {
+            hipLaunchKernelGGL((k_spectrum_rows<MAXH, 2, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_spectrum_rows<MAXH, 4, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+}
 template <typename C> static void launch_rows(gev_ctx *c, const PkArgsT<C> &A, int nblk, size_t shm) {
     const int h = c->N / 2 + 1;
-    if (h <= 65) hipLaunchKernelGGL((k_spectrum_rows<65, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
-    else if (h <= 257) hipLaunchKernelGGL((k_spectrum_rows<257, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
-    else hipLaunchKernelGGL((k_spectrum_rows<513, C>), dim3(nblk), dim3(TPB), shm, c->stream, A);
+    if (h <= 65) launch_rows_of<65>(c, A, nblk, shm);
+    else if (h <= 257) launch_rows_of<257>(c, A, nblk, shm);
+    else if (h <= 385) launch_rows_of<385>(c, A, nblk, shm);
+    else launch_rows_of<513>(c, A, nblk, shm);
 }
 
 // The spectrum with its device scratch given: the two tables (2N doubles),
