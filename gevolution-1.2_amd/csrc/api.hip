@@ -202,7 +202,7 @@ static void slab_layout(gev_ctx *c, const Sizes &s, SlabLayout &L) {
     L.add((void **)&c->scan_part, s.nblk_scan * 4);
     L.add((void **)&c->sort_segs, (s.n3 / 256 + 1) * 4);
     L.add((void **)&c->sort_big, sort_big_cap(s.cap) * 4);
-    L.add((void **)&c->sort_n, 8);
+    L.add((void **)&c->sort_n, 4);
     L.add((void **)&c->red_d, s.nred * 8);
     L.add((void **)&c->red_u, 64);
     c->pk_bins = spectrum_bins_cap(c->N);

@@ -92,16 +92,14 @@ __global__ __launch_bounds__(TPB) void k_cycle_begin(BoxCycle *__restrict__ cyc,
     c.dtd = c.dtau;
 }
 
-// The start of the particle stage: clears each box's kick maximum and filing
-// list counter (a box that stops after its field stage keeps the maximum of
-// its last kick, as the single-box driver does).
+// The start of the particle stage: clears each box's kick maximum (a box that
+// stops after its field stage keeps that of its last kick, as the single-box
+// driver does).
 __global__ __launch_bounds__(TPB) void k_particle_begin(const BoxCycle *__restrict__ cyc, int nbox, int64_t stride,
-                                                        unsigned long long *vmax0, uint32_t *sortn0) {
+                                                        unsigned long long *vmax0) {
     const int b = blockIdx.x * TPB + threadIdx.x;
     if (b >= nbox || !cyc[b].on) return;
     *box_ptr(vmax0, stride, b) = 0ull;
-    uint32_t *sn = box_ptr(sortn0, stride, b);
-    sn[0] = sn[1] = 0u;
 }
 
 // The end of the cycle (main.cpp:814, 867-874): the second half RK4 step,
@@ -298,7 +296,7 @@ int particle_stage(gev_batch *B) {
     gev_ctx *c = B->base;
     const Batch all{c->stride, B->cyc_d, 0};
     hipLaunchKernelGGL(k_particle_begin, dim3((c->nbox + TPB - 1) / TPB), dim3(TPB), 0, c->stream, B->cyc_d, c->nbox,
-                       c->stride, reinterpret_cast<unsigned long long *>(c->red_u), c->sort_n);
+                       c->stride, reinterpret_cast<unsigned long long *>(c->red_u));
     int rc = launch_particles_batch(c, B->gr != 0, all);
     if (rc) return rc;
     hipLaunchKernelGGL(k_cycle_end, dim3((c->nbox + TPB - 1) / TPB), dim3(TPB), 0, c->stream, B->cyc_d, c->nbox, c->N);

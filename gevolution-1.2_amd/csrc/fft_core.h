@@ -194,8 +194,8 @@ template <typename C, int L, int LINES, int NT> struct ColumnTile {
             for (int r = 0; r < R1; r++) x[r] = cconj(x[r]);
         }
     }
-    // the first stage into LDS (of the conjugate if CONJ); v is free afterwards (the caller may start
-    // the next tile's loads) and the caller synchronises before finish()
+    // the first stage into LDS (of the conjugate if CONJ); the caller
+    // synchronises before finish()
     template <bool CONJ> __device__ __forceinline__ void first(C *lds) {
 #pragma unroll
         for (int t = 0; t < J1; t++) {

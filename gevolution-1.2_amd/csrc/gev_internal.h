@@ -181,7 +181,7 @@ struct gev_ctx {
     uint32_t *scan_part = nullptr;  // scan block partials
     // the filing's ID sort: a flag byte per segment (256 consecutive cells)
     // with a cell of more than 4 particles, the listed cells of dense
-    // segments, and their count (sort_n[1])
+    // segments, and their count
     uint32_t *sort_segs = nullptr, *sort_big = nullptr, *sort_n = nullptr;
     int64_t scan_nblk = 0;
 

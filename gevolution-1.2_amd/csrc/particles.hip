@@ -1284,7 +1284,7 @@ static int finish_filing(gev_ctx *ctx, const Batch &bt = Batch{}) {
         if (scanned)
             hipLaunchKernelGGL(k_scan_partials, dim3(1, nb), dim3(TPB), 0, ctx->stream, ctx->scan_part, nblk, bt);
         hipLaunchKernelGGL(k_scan_final, dim3((unsigned)nblk, nb), dim3(TPB), 0, ctx->stream, ctx->count,
-                           n3v, ctx->scan_part, scanned, ctx->start, ctx->sort_n + 1, bt);
+                           n3v, ctx->scan_part, scanned, ctx->start, ctx->sort_n, bt);
     }
     if (ctx->n > 0) {
         ScopedTimer t(ctx, "filing_scatter");
@@ -1309,13 +1309,13 @@ static int finish_filing(gev_ctx *ctx, const Batch &bt = Batch{}) {
         const unsigned nsw = std::max((nseg + SORT_SEG_BATCH - 1) / SORT_SEG_BATCH, std::min(nseg, full));
         hipLaunchKernelGGL(k_sort_segments, dim3(nsw, nb), dim3(TPB), 0, ctx->stream, ctx->start, ctx->id, n3v,
                            ctx->perm, reinterpret_cast<const uint8_t *>(ctx->sort_segs),
-                           (uint32_t)grid_for(n3v, TPB), ctx->sort_big, ctx->sort_n + 1, ctx->id2, bt);
+                           (uint32_t)grid_for(n3v, TPB), ctx->sort_big, ctx->sort_n, ctx->id2, bt);
     }
     {
         ScopedTimer t(ctx, "filing_sort_dense_cells");
         // (1024 workgroups in all, at least 32 per box: 48 boxes of 32^3 had 49152)
         hipLaunchKernelGGL(k_sort_big, dim3(std::max(1024u / nb, 32u), nb), dim3(TPB), 0, ctx->stream, ctx->start,
-                           ctx->id, ctx->perm, ctx->sort_big, ctx->sort_n + 1, ctx->id2, bt);
+                           ctx->id, ctx->perm, ctx->sort_big, ctx->sort_n, ctx->id2, bt);
     }
     const int rc = check_hip(ctx, hipGetLastError(), "filing launch");
     if (!rc) ctx->count_clean = true;  // the scatter counted every cell back to zero
@@ -1339,9 +1339,9 @@ int launch_refile(gev_ctx *ctx) {
 
 // The particle stage over the boxes of a batch: kick + drift of every box
 // (its live set in, the other set out, its coefficients from its BoxCycle),
-// then the filing.  No clearing here: the batch clears vmax and the sort
-// list counter of every box before this stage, and every completed filing
-// leaves the counts at zero.
+// then the filing.  No clearing here: the batch clears vmax of every box
+// before this stage, the scan clears the sort's list counter, and every
+// completed filing leaves the counts at zero.
 int launch_particles_batch(gev_ctx *ctx, bool gr, const Batch &bt) {
     StepArgs sa{};
     if (ctx->n > 0) {
