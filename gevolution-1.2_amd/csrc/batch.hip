@@ -335,15 +335,23 @@ int run_stage(gev_batch *B, bool use_graph, bool fields) {
 
 // ---------------------------------------------------------------- autotuner
 //
-// The strided FFT passes (four y and four z passes per cycle and component
-// class) transform N-point columns staged W at a time; W (the tile's row
-// bytes) trades the occupancy of a workgroup against whole cache lines per
-// row, and the best choice depends on N and on how many boxes share the
-// launch.  The tuner times each candidate tile (64-, 128- and 256-byte rows)
-// on the batch's own FFT scratch field over every box, and keeps the
-// fastest per axis.  Every column is transformed the same way whatever the
-// tile, so the pick changes no result.  Picks are kept per (N, form, nbox)
-// for the process.
+// The strided FFT passes (per cycle four y launches, of one, six, one and four
+// components of every box; the cycle's z passes are those of the solves)
+// transform N-point columns staged W at a time; W (the tile's row bytes)
+// trades the occupancy of a workgroup against whole cache lines per row, and
+// the best choice depends on N and on how many boxes share the launch.  The
+// tuner times each candidate tile (64-, 128- and 256-byte rows) on the batch's
+// own FFT scratch field over every box, and keeps the fastest per axis.  Every
+// column is transformed the same way whatever the tile, so the pick changes no
+// result.  Picks are kept per (N, form, nbox) for the process.
+//
+// One component stands for the launches of several (their fields hold what the
+// caller may have put there): where its times are close, so are the cycles.
+// us per cycle with 64 / 128 / 256 bytes, and picked: 48 boxes of 32^3 FP64
+// 652 / 636 / 632, 632; 16 of 64^3 FP32 896 / 890 / 898, 892; 8 of 96^3 FP64
+// 2150 / 2131 / 2130, 2134 to 2155; 8 of 128^3 FP64 4894 / 4868 / 4859, 4858
+// to 4902; 4 of 192^3 FP32 5300 / 5275 / 5274, 5297; 4 of 256^3 FP32 11710 /
+// 11616 / 11646, 11626.  A pick has cost 1% at most.
 
 constexpr int TUNE_RB[3] = {64, 128, 256};
 
