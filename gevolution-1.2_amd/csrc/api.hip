@@ -33,20 +33,22 @@ static hipEvent_t take_event(gev_ctx *ctx) {
     return e;
 }
 
-void timer_begin(gev_ctx *ctx, const char *name) {
-    if (!ctx->timing) return;
+int timer_begin(gev_ctx *ctx, const char *name) {
+    if (!ctx->timing) return -1;
     TimerRec r;
     r.name = name;
     r.beg = take_event(ctx);
     r.end = take_event(ctx);
-    if (!r.beg || !r.end) return;
+    if (!r.beg || !r.end) return -1;
     (void)hipEventRecord(r.beg, ctx->stream);
     ctx->pending.push_back(r);
+    return (int)ctx->pending.size() - 1;
 }
 
-void timer_end(gev_ctx *ctx) {
-    if (!ctx->timing || ctx->pending.empty()) return;
-    (void)hipEventRecord(ctx->pending.back().end, ctx->stream);
+// (timers nest: an end recorded into the last record instead would leave the
+// outer one without, and its elapsed time an error for the next launch check)
+void timer_end(gev_ctx *ctx, int rec) {
+    if (rec >= 0) (void)hipEventRecord(ctx->pending[rec].end, ctx->stream);
 }
 
 static void timers_collect(gev_ctx *ctx) {

@@ -222,13 +222,14 @@ int fail(gev_ctx *ctx, int code, const std::string &msg);
 int check_hip(gev_ctx *ctx, hipError_t e, const char *what);
 
 // launch bracketing for the -DBENCHMARK style timers
-void timer_begin(gev_ctx *ctx, const char *name);
-void timer_end(gev_ctx *ctx);
+int timer_begin(gev_ctx *ctx, const char *name);  // the record timer_end closes, or -1
+void timer_end(gev_ctx *ctx, int rec);
 
 struct ScopedTimer {
     gev_ctx *c;
-    ScopedTimer(gev_ctx *ctx, const char *name) : c(ctx) { timer_begin(ctx, name); }
-    ~ScopedTimer() { timer_end(c); }
+    int rec;
+    ScopedTimer(gev_ctx *ctx, const char *name) : c(ctx), rec(timer_begin(ctx, name)) {}
+    ~ScopedTimer() { timer_end(c, rec); }
 };
 
 inline int64_t n3(const gev_ctx *c) { return (int64_t)c->N * c->N * c->N; }
