@@ -339,19 +339,21 @@ int run_stage(gev_batch *B, bool use_graph, bool fields) {
 // components of every box; the cycle's z passes are those of the solves)
 // transform N-point columns staged W at a time; W (the tile's row bytes)
 // trades the occupancy of a workgroup against whole cache lines per row, and
-// the best choice depends on N and on how many boxes share the launch.  The
-// tuner times each candidate tile (64-, 128- and 256-byte rows) on the batch's
-// own FFT scratch field over every box, and keeps the fastest per axis.  Every
-// column is transformed the same way whatever the tile, so the pick changes no
-// result.  Picks are kept per (N, form, nbox) for the process.
-//
-// One component stands for the launches of several (their fields hold what the
-// caller may have put there): where its times are close, so are the cycles.
-// us per cycle with 64 / 128 / 256 bytes, and picked: 48 boxes of 32^3 FP64
-// 652 / 636 / 632, 632; 16 of 64^3 FP32 896 / 890 / 898, 892; 8 of 96^3 FP64
-// 2150 / 2131 / 2130, 2134 to 2155; 8 of 128^3 FP64 4894 / 4868 / 4859, 4858
-// to 4902; 4 of 192^3 FP32 5300 / 5275 / 5274, 5297; 4 of 256^3 FP32 11710 /
-// 11616 / 11646, 11626.  A pick has cost 1% at most.
+// the best choice depends on N and on how many boxes and components share the
+// launch.  The tuner times each candidate tile (64-, 128- and 256-byte rows)
+// over every box and keeps the fastest per axis: the y pass by the four
+// launches of a cycle, on the FFT scratch and on SijFT, whose contents are put
+// aside meanwhile (by one launch on the FFT scratch where memory for that is
+// short), the z pass by one launch on the FFT scratch.  Every column is
+// transformed the same way whatever the tile, so the pick changes no result.
+// Picks are kept per (N, form, nbox) for the process.
+// us per cycle with 64 / 128 / 256 bytes, and with the pick: 48 boxes of 32^3
+// FP64 652 / 636 / 632, 636; 16 of 64^3 FP32 896 / 890 / 898, 900; 8 of 96^3
+// FP32 1434 / 1423 / 1406, 1413, FP64 2150 / 2131 / 2130, 2140; 8 of 128^3 FP64
+// 4894 / 4868 / 4859, 4875; 4 of 192^3 FP32 5300 / 5275 / 5274, 5279; 4 of
+// 256^3 FP32 11710 / 11616 / 11646, 11676.  (Picked by a launch of one
+// component: 96^3 FP32 1436, 128^3 4896, 192^3 5323; of six: 32^3 658, 96^3
+// FP64 2155.)
 
 constexpr int TUNE_RB[3] = {64, 128, 256};
 
@@ -388,23 +390,46 @@ int autotune(gev_batch *B) {
     const Batch all{c->stride, on, 0};
     const bool timing = c->timing;
     c->timing = false;
+    const size_t kept = 6 * (size_t)nk(c) * cbytes(c);
+    char *aside = nullptr;
+    if (!rc && hipMalloc(&aside, kept * c->nbox) != hipSuccess) {
+        aside = nullptr;
+        (void)hipGetLastError();
+    }
+    auto put = [&](bool back) {
+        for (int b = 0; b < c->nbox && aside && !rc; b++) {
+            double2 *const f = box_ptr(c->SijFT, c->stride, b);
+            char *const k = aside + b * kept;
+            rc = batch_hip(B, hipMemcpyAsync(back ? (void *)f : k, back ? (void *)k : f, kept, hipMemcpyDeviceToDevice,
+                                             c->stream), "tuner fields");
+        }
+    };
+    put(false);
     int best[2] = {0, 0};
     for (int axis = 0; axis < 2 && !rc; axis++) {
         float best_ms = 0.f;
         for (int v = 0; v < 3 && !rc; v++) {
             c->col_rb[axis] = TUNE_RB[v];
             auto pass = [&]() {
-                return axis == 0 ? fft_forward_y(c, c->fft_tmp, 1, all) : fft_forward_z(c, c->fft_tmp, 1, all);
+                if (axis == 1) return fft_forward_z(c, c->fft_tmp, 1, all);
+                int rp = fft_forward_y(c, c->fft_tmp, 1, all);
+                if (!aside) return rp;
+                if (!rp) rp = fft_forward_y(c, c->SijFT, 6, all);
+                if (!rp) rp = fft_forward_y(c, c->fft_tmp, 1, all);
+                return rp ? rp : fft_forward_y(c, c->SijFT, B->gr ? 4 : 1, all);
             };
             rc = pass();  // first use of the variant, untimed
-            if (!rc) rc = batch_hip(B, hipEventRecord(e0, c->stream), "tuner event");
-            for (int r = 0; r < 3 && !rc; r++) rc = pass();
-            if (!rc) rc = batch_hip(B, hipEventRecord(e1, c->stream), "tuner event");
-            if (!rc) rc = batch_hip(B, hipEventSynchronize(e1), "tuner sync");
-            float ms = 0.f;
-            if (!rc) rc = batch_hip(B, hipEventElapsedTime(&ms, e0, e1), "tuner time");
-            ms /= 3.f;
-            B->tune_ms[axis][v] = ms;
+            float ms = 0.f;  // the best of three
+            for (int r = 0; r < 3 && !rc; r++) {
+                rc = batch_hip(B, hipEventRecord(e0, c->stream), "tuner event");
+                if (!rc) rc = pass();
+                if (!rc) rc = batch_hip(B, hipEventRecord(e1, c->stream), "tuner event");
+                if (!rc) rc = batch_hip(B, hipEventSynchronize(e1), "tuner sync");
+                float t = 0.f;
+                if (!rc) rc = batch_hip(B, hipEventElapsedTime(&t, e0, e1), "tuner time");
+                if (r == 0 || t < ms) ms = t;
+            }
+            B->tune_ms[axis][v] = ms / (axis == 0 && aside ? 8 + (B->gr ? 4 : 1) : 1);  // per component
             if (!rc && (v == 0 || ms < best_ms)) {
                 best_ms = ms;
                 best[axis] = TUNE_RB[v];
@@ -413,6 +438,11 @@ int autotune(gev_batch *B) {
         c->col_rb[axis] = best[axis];
     }
     c->timing = timing;
+    put(true);
+    if (aside) {
+        if (!rc) rc = batch_hip(B, hipStreamSynchronize(c->stream), "tuner fields");
+        (void)hipFree(aside);
+    }
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (on) (void)hipFree(on);
