@@ -76,7 +76,7 @@ template <int N, int KIND, typename C> constexpr int zs_cols() {
 // input transform where the registers allow it; at N = 384 and above 512 the
 // prefetch would spill, and at N = 192 it would leave one wave per SIMD
 // (compiler resource report), so B is read at the solve.  (us per launch at
-// 192^3, prefetched -> read: FP64 393 -> 287, FP32 253 -> 184; FP32 form at
+// 192^3, prefetched -> read: FP64 384 -> 296, FP32 253 -> 185; FP32 form at
 // 512^3, where it fits: 3.04 against 3.21 ms with B read at the solve.)
 #ifndef GEV_ZS_AHEAD
 #define GEV_ZS_AHEAD 1
@@ -345,9 +345,10 @@ __global__ __launch_bounds__((zs_threads<N, KIND, C>())) void k_zsolve(ZArgsT<C>
 // components; half as many barriers as k_zsolve, and two components' loads in
 // flight.
 // Bound by the latency of its loads and barriers at 8 waves per CU (the
-// registers; 3.7 TB/s at 512^3).  us per launch, k_zsolve -> this: 512^3 4756
-// -> 4685, 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.9 -> 16.5, 32^3 12.1
-// both.  FP32 stays on k_zsolve: its float points leave a thread room for 8
+// registers; 3.7 TB/s at 512^3, where 52% of the wave cycles wait and 20%
+// issue).  us per launch, k_zsolve -> this: 512^3 4704 -> 4701 to 4756 -> 4685
+// (run by run), 256^3 603 -> 589, 128^3 78.7 -> 71.9, 64^3 20.9 -> 16.5, 32^3
+// 12.1 both.  FP32 stays on k_zsolve: its float points leave a thread room for 8
 // points of all components only with spills (512^3 3012 -> 3432, 256^3 344 ->
 // 572); so do the FP64 solves with fewer fields, which gain nothing (Poisson
 // 512^3 620 -> 636, chi alone 256^3 294 -> 305).  The solve of a point stands in
