@@ -558,9 +558,11 @@ template <typename F, typename C> struct XArgsT {
 using XArgs = XArgsT<double, double2>;
 
 // NC: 1 the scalar source, 6 the tensor's components in one workgroup (phi
-// is read once for all), TENSOR_ONE the tensor with one component per
-// workgroup (blockIdx.z), for grids whose rows would not fill the chip.
-constexpr int TENSOR_ONE = -6;
+// is read once for all), TENSOR_WIDE the same over up to twice the rows,
+// TENSOR_ONE the tensor with one component per workgroup (blockIdx.z), for
+// grids whose rows would not fill the chip.
+constexpr int TENSOR_ONE = -6, TENSOR_WIDE = 7;
+constexpr bool tensor_six(int NC) { return NC == 6 || NC == TENSOR_WIDE; }
 
 // Rows per workgroup: the NC prepared components of a thread's points are
 // held in registers until each is transformed, so the 6-component form
@@ -570,6 +572,7 @@ constexpr int TENSOR_ONE = -6;
 #endif
 template <int N, int NC> constexpr int xprep_lines() {
     int l = x_lines<N>();
+    while (NC == TENSOR_WIDE && l * N <= 2048) l *= 2;
     while (NC == TENSOR_ONE && l > 1 && l * (N / 2) > 512) l /= 2;
     while (NC > 1 && l > 1 && l * (N / 2) > GEV_XPREP_PTS * 256) l /= 2;
     return l;
@@ -579,7 +582,7 @@ template <int N, int NC, typename F, typename C>
 __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
     using R = decltype(C::x);
     constexpr int TPB = 256;
-    constexpr int NV = NC == 6 ? 6 : 1;  // components of this workgroup
+    constexpr int NV = tensor_six(NC) ? 6 : 1;  // components of this workgroup
     constexpr int M = N / 2;
     constexpr int LINES = xprep_lines<N, NC>();
     constexpr int PER = (LINES * M + TPB - 1) / TPB;
@@ -624,7 +627,7 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
             const int x = 2 * n + h;
             const int64_t i = row * N + x;
             const Nb c = nb_of(x, y, z, N);
-            if constexpr (NC == 6) {
+            if constexpr (tensor_six(NC)) {
                 F T[6], S[6];
 #pragma unroll
                 for (int q = 0; q < 6; q++) T[q] = A.src[q * A.n3v + i];
@@ -672,9 +675,28 @@ __global__ __launch_bounds__(256) void k_r2c_x_prep(XArgsT<F, C> A) {
 template <int N, int NC, typename F, typename C> int launch_x(gev_ctx *c, const XArgsT<F, C> &A) {
     constexpr int LINES = xprep_lines<N, NC>();
     const unsigned nbox = A.bt.cyc ? (unsigned)c->nbox : 1u;
-    // A tensor pass of fewer workgroups than two per CU takes one component in
-    // each instead, which re-reads phi from L2 (64^3: 15.9 -> 11.8 us, 32^3:
-    // 13.4 -> 7.4; 96^3, 576 workgroups: equal; 128^3, 1024: 61 -> 80)
+    // Twice the rows per workgroup in FP64 below 128^3 where that takes fewer
+    // rounds of the chip: a CU holds four workgroups of up to 512 points or
+    // three of twice that (registers), a round of which takes 4/3 of the time
+    // (a tie goes to the latter at the radix-3 sizes, 768 points).  us, up to
+    // 512 points -> twice that: 48 boxes of 32^3 44.7 -> 37.8, 6 of 64^3 42.7 ->
+    // 39.3, 12 79.7 -> 78.5, 64 of 24^3 29.1 -> 27.4, 24 of 48^3 76.3 -> 72.6, 8
+    // of 96^3 197 -> 193; not taken: 32 of 32^3 27.3 -> 29.3, 4 of 64^3 25.7 ->
+    // 31.3, 8 52.4 -> 56.5, 16 105.5 -> 106.9, 12 of 48^3 40.0 -> 42.3, 256 of
+    // 16^3 30.1 -> 33.6, 128^3 54.8 -> 60.0, and FP32, 16 of 64^3, 62.4 -> 68.0.
+    if constexpr (NC == 6 && N >= 24 && N < 128 && sizeof(F) == 8) {
+        constexpr int L2 = xprep_lines<N, TENSOR_WIDE>();
+        const unsigned wide = gev::grid_for(A.nrows, L2) * nbox, narrow = gev::grid_for(A.nrows, LINES) * nbox;
+        const unsigned tie = L2 * N / 2 < 1024 ? 1 : 0;
+        if (wide >= 512 && 4 * ((wide + 767) / 768) < 3 * ((narrow + 1023) / 1024) + tie) {
+            hipLaunchKernelGGL((k_r2c_x_prep<N, TENSOR_WIDE, F, C>), dim3(gev::grid_for(A.nrows, L2), nbox), dim3(256),
+                               0, c->stream, A);
+            return gev::check_hip(c, hipGetLastError(), "fused x pass launch");
+        }
+    }
+    // One of fewer workgroups than two per CU takes one component in each
+    // instead, which re-reads phi from L2 (64^3, 128 workgroups of 1024 points:
+    // 15.9 -> 11.8 us, 32^3: 13.4 -> 7.4; 96^3, 576: equal; 128^3, 1024: 61 -> 80)
     if constexpr (NC == 6 && N <= 128) {
         constexpr int L1 = xprep_lines<N, TENSOR_ONE>();
         if (gev::grid_for(A.nrows, LINES) * nbox < 512) {

@@ -1,7 +1,8 @@
 """Batches at the sizes where the launches over boxes take another path than a
 small batch's: the z pass that solves on registers with boxes (FP64, 64^3 and
 128^3), the tensor x pass with six components per workgroup and boxes (32^3
-from 16 boxes on, 96^3), one component per workgroup just below that line,
+from 16 boxes on, 96^3; over twice the rows with 40 boxes of 32^3, 57 of 24^3, 8
+of 48^3, 5 of 64^3), one component per workgroup just below that line,
 column passes over components and boxes, radix-3 grids.  Boxes of different
 states, one stopped after the first cycle, graph replay and plain launches:
 every carried field and the particles of each equal those of the box run
@@ -34,7 +35,7 @@ def fill(gev, box, s, i):
 
 
 @pytest.mark.parametrize("N,nbox,form,gr", [
-    (32, 15, 0, 1), (32, 17, 0, 1), (32, 17, 1, 1), (32, 66, 1, 0), (48, 3, 0, 1), (64, 3, 0, 1), (64, 2, 1, 1),
+    (32, 15, 0, 1), (32, 17, 0, 1), (32, 17, 1, 1), (32, 66, 1, 0), (32, 40, 0, 1), (24, 57, 0, 1), (48, 3, 0, 1), (48, 8, 0, 1), (64, 5, 0, 1), (64, 3, 0, 1), (64, 2, 1, 1),
     (96, 2, 0, 1), (96, 2, 1, 1), (128, 2, 0, 1), (192, 2, 0, 1)])
 def test_boxes_equal_alone(gev, N, nbox, form, gr):
     s = gr_state(N, N + nbox)

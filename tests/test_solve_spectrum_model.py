@@ -169,9 +169,9 @@ def x_lines(N):
 
 @pytest.mark.parametrize("N", SIZES)
 def test_prepared_rows(N):
-    """Rows per workgroup of the scalar, the six-component and the
-    one-component form: the registers a thread holds, the LDS of the padded
-    lines, and every row taken."""
+    """Rows per workgroup of the scalar, the six-component (over up to twice
+    the rows too) and the one-component form: the registers a thread holds,
+    the LDS of the padded lines, and every row taken."""
     M = N // 2
     six = x_lines(N)
     while six > 1 and six * M > PTS * 256:
@@ -179,7 +179,13 @@ def test_prepared_rows(N):
     one = x_lines(N)
     while one > 1 and one * M > 512:
         one //= 2
-    for lines in (x_lines(N), six, one):
+    wide = x_lines(N)
+    while wide * N <= 2048:
+        wide *= 2
+    while wide > 1 and wide * M > PTS * 256:
+        wide //= 2
+    assert six <= wide <= 4 * six and wide * M <= 1024
+    for lines in (x_lines(N), six, wide, one):
         assert lines >= 1 and -(-N * N // lines) * lines >= N * N
         assert (lines * (M + M // 16) + M) * 16 <= 64 * 1024
     assert six * M <= PTS * 256 and (one * M <= 512 or one == 1)
